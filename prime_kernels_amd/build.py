@@ -17,7 +17,8 @@ PKG = Path(__file__).resolve().parent
 ROOT = PKG.parent
 LIB_DIR = PKG / "_lib"
 LIB = LIB_DIR / "libprime_decode.so"
-SOURCES = [PKG / "csrc" / "decode_megakernel.hip", PKG / "csrc" / "decode_sr.hip", PKG / "csrc" / "lossless_bf16.hip"]
+SOURCES = [PKG / "csrc" / "decode_megakernel.hip", PKG / "csrc" / "decode_sr.hip", PKG / "csrc" / "decode_cell.hip",
+           PKG / "csrc" / "lossless_bf16.hip"]
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [

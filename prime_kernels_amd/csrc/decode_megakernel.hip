@@ -1,6 +1,7 @@
 // SmolLM2 single-token decode step as one persistent HIP kernel per step for gfx950 (MI355X): the
-// general batch-1 kernel (decode_kernel) and the batched kernel (decode_kernel_b); the split-role
-// batch-1 kernel is in decode_sr.hip.  The launch is an ordinary hipLaunchKernel of one workgroup
+// general batch-1 kernel (decode_kernel) and the batched kernel of two sequences with per-layer outputs
+// or stage capture, and of given hidden states (decode_kernel_b); the split-role batch-1 kernel is in
+// decode_sr.hip, the kernel of three or more sequences in decode_cell.hip.  The launch is an ordinary hipLaunchKernel of one workgroup
 // per CU, which relies on all 256 workgroups being resident at once (true on an otherwise idle
 // device: a workgroup waiting for one that is not resident gives up after its bounded wait and the
 // step comes back poisoned and reported); PK_LAUNCH=cooperative or pk_set_option(PK_OPT_COOPERATIVE)
@@ -3211,7 +3212,8 @@ static constexpr size_t ws_general_bytes() {
 static constexpr size_t rec_general_bytes() {
   return round_up((WS<G360>::XREC_WORDS > WS<G135>::XREC_WORDS ? WS<G360>::XREC_WORDS : WS<G135>::XREC_WORDS) * 4, 4096);
 }
-static size_t ws_bytes() { return ws_general_bytes() + round_up(sr_region_bytes(1), 4096); }
+static size_t cell_region_off() { return ws_general_bytes() + round_up(sr_region_bytes(1), 4096); }
+static size_t ws_bytes() { return cell_region_off() + round_up(cell_region_bytes(), 4096); }
 // the split-role group-A records: the narrow layout's, then the wide layout's (separate lines, so
 // that no XCD's L2 holds a line another layout writes from another XCD)
 static size_t rec_wide_off() { return rec_general_bytes() + round_up(sr_local_bytes(0), 4096); }
@@ -3513,9 +3515,8 @@ static int decode_impl(void* stream, int B, int n_layers, const void* input_ids,
     if (B > 1) {
       if (B == 2 && opt_split_role() && !input_hidden && !layer_outputs) {
         // two sequences: each as a batch-1 step of its own, on the split-role kernel.  Two such steps
-        // take less time than one batched step of two (360M, contexts drawn from 128..4096: 1.03
-        // against 1.42 ms); from three sequences on, the batched kernel, which reads the weights
-        // once for all of them, is faster (1.39 ms at three)
+        // take less time than one step of two on decode_kernel_b (360M, contexts drawn from 128..4096:
+        // 1.03 against 1.42 ms)
         for (int b = 0; b < 2; ++b) {
           Params q = p;
           q.B = 1;
@@ -3532,6 +3533,11 @@ static int decode_impl(void* stream, int B, int n_layers, const void* input_ids,
         }
         return PK_OK;
       }
+      // three or more: cells of XCDs, each decoding its own sequences (360M, three sequences of 100..2000
+      // tokens: 748 us against 1,329 here); two with layer_outputs and given hidden states stay here
+      if (B > 2 && !input_hidden)
+        return cell_launch(G::H == 960 ? PK_MODEL_SMOLLM2_360M : PK_MODEL_SMOLLM2_135M, p,
+                           reinterpret_cast<const uint8_t*>(state->ws) + cell_region_off(), s, opt_cooperative());
       return launch<G, true>(p, s);
     }
   return batch1(p);
