@@ -198,6 +198,10 @@ size_t pk_mxfp8_scale_stride(int cols);
  * the rule prime_kernels/rmsnorm/test.cu:126-144 applies.  q [rows, cols], scales
  * [rows, pk_mxfp8_scale_stride(cols)]; all pointers 16-byte aligned. */
 int pk_quantize_mxfp8(void* stream, const void* src, void* q, void* scales, int rows, int cols);
+/* The same for n matrices in one launch (host arrays of n entries): nothing is launched when any of
+ * them is refused. */
+int pk_quantize_mxfp8_many(void* stream, int n, const void* const* src, void* const* q, void* const* scales,
+                           const int* rows, const int* cols);
 
 /* Device properties relevant to the launch (current device). Returns a status. */
 int pk_query(int* cu_count, int* coop, int* max_lds_per_block, int* is_gfx950, size_t* lds_bytes);

@@ -52,6 +52,15 @@ int lossless_encode_layer(const void* input, void* plane, void* headers, void* r
                           void* flags, void* prefix, void* scan_workspace, size_t scan_workspace_bytes,
                           void* enabled, uint32_t capacity, void* stream);
 
+/* Encode `layers` matrices, 32 a launch (host arrays of one entry per layer, the buffers as above);
+ * totals [layers] receives each layer's escaped chunks.  Nothing is launched when a layer is refused.
+ * No reference counterpart. */
+size_t lossless_encode_workspace_bytes(int layers);
+int lossless_encode_layers(int layers, const void* const* input, void* const* plane, void* const* headers,
+                           void* const* raw, void* const* row_offsets, void* const* enabled,
+                           const uint32_t* capacity, void* totals, void* workspace, size_t workspace_bytes,
+                           void* stream);
+
 /* Decode one encoded matrix back to bf16 [5120, 960] (bit-exact).  Only for a matrix whose enabled
  * flag is 1: a disabled one has escape ordinals past its table. */
 int lossless_decode_layer(const void* plane, const void* headers, const void* raw, void* output, void* stream);

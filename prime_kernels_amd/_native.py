@@ -51,6 +51,7 @@ SIGNATURES = {
                              ll, ll, ll, ll, ll, ci, vp, ci, vp, vp, vp, vp, vp, sz, ci]),
     "pk_mxfp8_scale_stride": (sz, [ci]),
     "pk_quantize_mxfp8": (ci, [vp, vp, vp, vp, ci, ci]),
+    "pk_quantize_mxfp8_many": (ci, [vp, ci, vp, vp, vp, vp, vp]),
     "pk_query": (ci, [ctypes.POINTER(ci), ctypes.POINTER(ci), ctypes.POINTER(ci), ctypes.POINTER(ci),
                       ctypes.POINTER(sz)]),
     "prime_decode_status_string": (ctypes.c_char_p, [ci]),
@@ -72,6 +73,8 @@ SIGNATURES = {
     # include/prime_lossless.h
     "lossless_scan_workspace_bytes": (sz, []),
     "lossless_encode_layer": (ci, [vp, vp, vp, vp, vp, vp, vp, vp, sz, vp, ctypes.c_uint, vp]),
+    "lossless_encode_workspace_bytes": (sz, [ci]),
+    "lossless_encode_layers": (ci, [ci, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp]),
     "lossless_decode_layer": (ci, [vp, vp, vp, vp, vp]),
     "lossless_write_descriptor": (ci, [vp, ci, vp, vp, vp, vp, vp, vp]),
     "decode360_lossless": (ci, [vp, ci, vp, vp, vp, vp, vp, vp, ci, vp, vp, vp, ll, ll, ll, ll, ll, ci, vp, ci,

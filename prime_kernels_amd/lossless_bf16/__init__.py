@@ -7,8 +7,8 @@ an escape table of whole chunks, row offsets, and an enabled flag that the encod
 layer's escapes do not fit its table).
 
 Design.  All encoding, decoding and scanning runs in the library's HIP kernels on the cache's
-device.  An encoder pass launches every layer back to back and copies each layer's escape count
-to a device vector right behind its launch, so a pass costs one host synchronisation.  Preparation
+device.  An encoder pass encodes every layer in one launch, which also leaves the layers' escape
+counts in a device vector, so a pass costs one call and one host synchronisation.  Preparation
 is two passes: with empty tables (the encoder only counts, and disables every layer that has
 escapes), then with tables sized at HEADROOM times the count.  `refresh` is one pass into the
 existing tables; a layer that now has more escapes than its table holds stays disabled, and the
@@ -65,11 +65,9 @@ class EncodedGUCache:
         self._lib = _native.library()
         dev = self.device
         u32 = torch.uint32
-        # scratch shared by the layers of a pass (the encoder's chunk flags and their inclusive scan)
-        self._scan_bytes = self._lib.lossless_scan_workspace_bytes()
+        # the encoder's scratch: its scan states
+        self._scan_bytes = self._lib.lossless_encode_workspace_bytes(LAYERS)
         self._scan = torch.empty((self._scan_bytes,), dtype=torch.uint8, device=dev)
-        self._flags = torch.empty((CHUNKS,), dtype=u32, device=dev)
-        self._prefix = torch.empty((CHUNKS,), dtype=u32, device=dev)
         self._counts = torch.empty((LAYERS,), dtype=u32, device=dev)
         self._layers = [
             _LayerCode(plane=torch.empty((ROWS, COLS), dtype=torch.uint8, device=dev),
@@ -79,11 +77,13 @@ class EncodedGUCache:
                        enabled=torch.empty((), dtype=u32, device=dev))
             for _ in range(LAYERS)]
         self.table = torch.empty((LAYERS * DESCRIPTOR_BYTES,), dtype=torch.uint8, device=dev)
+        self._columns = None
         # pass 1 counts (no table has room), pass 2 encodes into tables with headroom
         counts = self._encode_pass(weights, [0] * LAYERS)
         for code, n in zip(self._layers, counts):
             code.capacity = max(1, math.ceil(n * HEADROOM))
             code.raw = torch.empty((code.capacity * 8,), dtype=torch.uint16, device=dev)
+        self._columns = None
         counts = self._encode_pass(weights, [c.capacity for c in self._layers])
         for code, n in zip(self._layers, counts):
             code.found = n
@@ -99,9 +99,10 @@ class EncodedGUCache:
     # -- the tensors the cache encodes ------------------------------------------------------------
 
     def _check(self, weights) -> None:
+        device, shape = self.device, torch.Size((ROWS, COLS))
         for i, t in enumerate(weights):
-            ok = (isinstance(t, torch.Tensor) and t.is_cuda and t.device == self.device and t.dtype == torch.bfloat16
-                  and tuple(t.shape) == (ROWS, COLS) and t.is_contiguous() and t.data_ptr() % 16 == 0)
+            ok = (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.bfloat16 and t.shape == shape
+                  and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0)
             if not ok:
                 raise ValueError(f"gate_up matrix {i}: need a contiguous, 16-byte aligned bf16 [{ROWS}, {COLS}] "
                                  f"tensor on {self.device}")
@@ -116,15 +117,21 @@ class EncodedGUCache:
     def _encode_pass(self, weights, capacities) -> list:
         """Encode every layer on the current stream; returns the escape chunks each layer has."""
         stream = torch.cuda.current_stream(self.device)
-        for i, (t, code) in enumerate(zip(weights, self._layers)):
-            _raise_on(self._lib.lossless_encode_layer(
-                t.data_ptr(), code.plane.data_ptr(), code.headers.data_ptr(), code.raw.data_ptr(),
-                code.row_offsets.data_ptr(), self._flags.data_ptr(), self._prefix.data_ptr(), self._scan.data_ptr(),
-                self._scan_bytes, code.enabled.data_ptr(), capacities[i], stream.cuda_stream), f"encode layer {i}")
-            # the scan total, copied before the next layer reuses the scan
-            self._counts[i:i + 1].copy_(self._prefix[CHUNKS - 1:])
-        stream.synchronize()
-        return [int(n) for n in self._counts.view(torch.int32).cpu().tolist()]
+        pointers = ctypes.c_void_p * LAYERS
+
+        def column(tensors):
+            return pointers(*[t.data_ptr() for t in tensors])
+
+        if self._columns is None:  # the cache's own buffers, until the escape tables are allocated again
+            codes = self._layers
+            self._columns = [column(c.plane for c in codes), column(c.headers for c in codes), column(c.raw for c in codes),
+                             column(c.row_offsets for c in codes), column(c.enabled for c in codes)]
+        with torch.cuda.device(self.device):
+            rc = self._lib.lossless_encode_layers(LAYERS, column(weights), *self._columns, (ctypes.c_uint32 * LAYERS)(*capacities),
+                                                  self._counts.data_ptr(), self._scan.data_ptr(), self._scan_bytes,
+                                                  stream.cuda_stream)
+        _raise_on(rc, "encode")
+        return self._counts.view(torch.int32).tolist()  # waits for the pass
 
     @torch.inference_mode()
     def refresh(self, weights) -> None:
@@ -156,7 +163,7 @@ class EncodedGUCache:
                 "enabled": c.enabled}
 
     def _owned(self):
-        yield from (self._scan, self._flags, self._prefix, self._counts, self.table)
+        yield from (self._scan, self._counts, self.table)
         for c in self._layers:
             yield from (c.plane, c.headers, c.raw, c.row_offsets, c.enabled)
 
