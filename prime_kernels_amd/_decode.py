@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+from array import array
 from dataclasses import dataclass
 
 import torch
@@ -93,7 +94,12 @@ class _Runtime:
         self.ids = torch.empty((model.max_batch,), dtype=torch.int64, device=device)
         self.layers_t = None
         self.kv_t = None
-        self.table_key = None
+        self.table_key = None   # the addresses in the tables, layers then caches, as bytes
+        self.spec = _native.host().make_spec(
+            model.model_id, model.hidden, model.kv_heads, model.head_dim, model.max_batch, model.max_seq, model.layers,
+            VOCAB, BLOCK_SIZE, [(dtype == torch.bfloat16, shape) for _, dtype, shape in model.layer_spec()])
+        self.entry = _native.entry_address("pk_decode_mxfp8" if model.weight_format == "mxfp8" else "pk_decode")
+        self.entry_encoded = _native.entry_address("pk_decode_lossless")
 
     def _stream(self, stream):
         return torch.cuda.current_stream(self.device).cuda_stream if stream is None else stream
@@ -160,21 +166,45 @@ def _check_tensor(tensor, name, *, dtype=None, device=None, shape=None):
         raise ValueError(f"{name} must have shape {shape}")
 
 
+def _set_tables(rt: _Runtime, key: bytes, n_layers: int) -> None:
+    """Put the addresses of `key` (every layer's tensors, then the caches) into the device tables."""
+    addresses = torch.frombuffer(bytearray(key), dtype=torch.int64)
+    layer_table, kv_table = addresses[:-n_layers].view(n_layers, -1), addresses[-n_layers:]
+    if rt.layers_t is None or rt.layers_t.shape != layer_table.shape:
+        rt.layers_t = layer_table.to(rt.device)
+        rt.kv_t = kv_table.to(rt.device)
+    else:
+        # in place, so graphs captured with these tables see the new pointers
+        rt.layers_t.copy_(layer_table)
+        rt.kv_t.copy_(kv_table)
+    rt.table_key = key
+
+
 def _tables(rt: _Runtime, layers, kv_caches):
     """Device pointer tables (reference: decode_megakernel_360m/__init__.py:126-139)."""
-    key = (tuple(t.data_ptr() for layer in layers for t in layer), tuple(t.data_ptr() for t in kv_caches))
+    key = array("q", [t.data_ptr() for layer in layers for t in layer] + [t.data_ptr() for t in kv_caches]).tobytes()
     if key != rt.table_key:
-        layer_table = torch.tensor([[t.data_ptr() for t in layer] for layer in layers], dtype=torch.int64)
-        kv_table = torch.tensor([t.data_ptr() for t in kv_caches], dtype=torch.int64)
-        if rt.layers_t is None or rt.layers_t.shape != layer_table.shape:
-            rt.layers_t = layer_table.to(rt.device)
-            rt.kv_t = kv_table.to(rt.device)
-        else:
-            # in place, so graphs captured with these tables see the new pointers
-            rt.layers_t.copy_(layer_table)
-            rt.kv_t.copy_(kv_table)
-        rt.table_key = key
+        _set_tables(rt, key, len(kv_caches))
     return rt.layers_t, rt.kv_t
+
+
+def _plain_step(rt: _Runtime, model: Model, nl: int, encoded_gu, want_ids, input_ids, positions, seq_lens, block_table,
+                slot_mapping, embed, layers, final_norm, kv_caches, cos_sin_cache, layer_outputs, logits_out):
+    """Check and launch in the host module: the entry point's status, or None when an argument is not
+    plainly right (decode_step's own checks then decide)."""
+    step, stream = _native.host().step, torch.cuda.current_stream(rt.device).cuda_stream
+    for _ in range(2):
+        r = step(rt.entry if encoded_gu is None else rt.entry_encoded, stream, rt.spec, nl, input_ids, positions, seq_lens,
+                 slot_mapping, block_table, embed, final_norm, layers, kv_caches, cos_sin_cache, layer_outputs, logits_out,
+                 want_ids, rt.out.data_ptr(), rt.ids.data_ptr(), rt.scratch_ptr, rt.scratch_bytes,
+                 rt.layers_t.data_ptr() if rt.layers_t is not None else None,
+                 rt.kv_t.data_ptr() if rt.kv_t is not None else None, rt.table_key,
+                 encoded_gu.table.data_ptr() if encoded_gu is not None else None,
+                 encoded_gu.weights if encoded_gu is not None else None)
+        if not isinstance(r, bytes):
+            return r
+        _set_tables(rt, r, nl)
+    return None
 
 
 def _failure_message(model: Model, rc: int) -> str:
@@ -211,6 +241,17 @@ def decode_step(model: Model, *, input_ids, positions, seq_lens, block_table, sl
     the same gate_up matrices, SmolLM2-360M only) makes the batch-1 step stream the encoded gate/up
     weights of every enabled layer."""
     nl = model.layers if num_layers is None else int(num_layers)
+    rt = _runtimes.get((model.name, input_ids.device)) if type(input_ids) is torch.Tensor else None
+    if rt is not None and debug is None and eps == EPS and -1 <= debug_layer_index < model.layers and (
+            encoded_gu is None or (model.model_id == 360 and model.weight_format == "bf16" and encoded_gu.device == rt.device)):
+        rc = _plain_step(rt, model, nl, encoded_gu, return_token_ids or logits_out is not None, input_ids, positions,
+                         seq_lens, block_table, slot_mapping, embed, layers, final_norm, kv_caches, cos_sin_cache,
+                         layer_outputs, logits_out)
+        if rc is not None:
+            if rc != 0:
+                raise RuntimeError(_failure_message(model, rc))
+            batch = input_ids.shape[0]
+            return (rt.out[:batch], rt.ids[:batch]) if return_token_ids else rt.out[:batch]
     batch = input_ids.shape[0]
     if not 1 <= batch <= model.max_batch:
         raise ValueError(f"batch must be 1..{model.max_batch}, got {batch}")

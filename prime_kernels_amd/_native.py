@@ -1,15 +1,19 @@
-"""ctypes binding of the C ABI in include/prime_decode.h (libprime_decode.so).
+"""ctypes binding of the C ABI in include/prime_decode.h (libprime_decode.so), and the host module
+that checks and launches a decode step (csrc/host_step.cpp).
 
-This is the only place Python crosses into native code.  There is no fallback: if the library
-is missing the import-time call raises.
+This is the only place Python crosses into native code.  There is no fallback: if either is
+missing its first use raises.
 """
 
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libprime_decode.so"
+HOST_PATH = LIB_PATH.with_name("_host_step.so")
 
 MODEL_360M = 360
 MODEL_135M = 135
@@ -25,6 +29,7 @@ PK_OPT_SKEW = 4
 PK_OPT_SPLIT_WIDE = 5
 
 _lib = None
+_host = None
 
 vp, ci, ll, sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_longlong, ctypes.c_size_t
 
@@ -100,3 +105,23 @@ def library() -> ctypes.CDLL:
 
 def status_string(rc: int) -> str:
     return library().prime_decode_status_string(rc).decode()
+
+
+def host():
+    """The host module: make_spec and step (csrc/host_step.cpp)."""
+    global _host
+    if _host is None:
+        if not HOST_PATH.is_file():
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -m prime_kernels_amd.build`")
+        import torch  # noqa: F401  (the module links against torch's libraries)
+
+        loader = importlib.machinery.ExtensionFileLoader("_host_step", str(HOST_PATH))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_host_step", loader))
+        loader.exec_module(module)
+        _host = module
+    return _host
+
+
+def entry_address(name: str) -> int:
+    """Address of a library entry point, for the host module."""
+    return ctypes.cast(getattr(library(), name), ctypes.c_void_p).value

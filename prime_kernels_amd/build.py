@@ -1,4 +1,5 @@
-"""Build the native library `_lib/libprime_decode.so` with hipcc for gfx950.
+"""Build the native library `_lib/libprime_decode.so` with hipcc for gfx950, and the host module
+`_lib/_host_step.so`.
 
 Usage: python -m prime_kernels_amd.build   (also called by __graft_entry__.build()).
 The library is built in-tree so it travels with the source tree; nothing is JIT-compiled at
@@ -11,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -19,6 +21,8 @@ LIB_DIR = PKG / "_lib"
 LIB = LIB_DIR / "libprime_decode.so"
 SOURCES = [PKG / "csrc" / "decode_megakernel.hip", PKG / "csrc" / "decode_sr.hip", PKG / "csrc" / "decode_cell.hip",
            PKG / "csrc" / "lossless_bf16.hip"]
+HOST_SOURCE = PKG / "csrc" / "host_step.cpp"
+HOST_LIB = LIB_DIR / "_host_step.so"
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [
@@ -48,7 +52,28 @@ def build(verbose: bool = False) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed ({res.returncode}):\n{res.stderr[-4000:]}")
     os.replace(tmp, LIB)
+    build_host(verbose)
     return LIB
+
+
+def build_host(verbose: bool = False) -> Path:
+    """The Python module of the step's argument checks (host code only), against the installed torch."""
+    import torch
+
+    torch_dir = Path(torch.__file__).resolve().parent
+    lib = torch_dir / "lib"
+    tmp = HOST_LIB.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX") or shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{torch_dir / 'include'}",
+           f"-I{torch_dir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}", f"-I{sysconfig.get_paths()['include']}",
+           str(HOST_SOURCE), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", f"-Wl,-rpath,{lib}", "-o", str(tmp)]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed ({res.returncode}):\n{res.stderr[-4000:]}")
+    os.replace(tmp, HOST_LIB)
+    return HOST_LIB
 
 
 if __name__ == "__main__":
