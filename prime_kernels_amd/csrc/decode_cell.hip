@@ -20,8 +20,8 @@
 // a ring), waves 4..7 consumers, as in the other decode kernels.  Ring packets are 1 KB: 8 rows x
 // 128 bytes, row r's 16-byte piece c in slot (c + r) mod 8, for weight rows and cached tokens alike,
 // so that an MFMA operand read touches 8 different bank groups with each 8 lanes.  A projection's
-// packets run k-step by k-step over all of the workgroup's rows; consumer wave w takes k-steps w,
-// w + 4, ..., so the waves use the stream as it lands, and one LDS reduction in wave order ends the
+// packets run k-step by k-step over all of the workgroup's rows; consumer wave w takes its quarter of the k-steps
+// into registers before the phase's input is waited for, and one LDS reduction, (w0 + w1) + (w2 + w3), ends the
 // phase (deterministic).
 //
 // Exchange format: 16-byte units {two 32-bit words of payload (four bf16, the four consecutive rows
@@ -55,8 +55,15 @@ constexpr uint32_t LDS_CU = 160u * 1024u;  // LDS of a CU (one workgroup each)
 #define PK_CELL_TMIN 8
 #endif
 constexpr int DEPTH_C = PK_CELL_DEPTH;     // packets in flight per producer wave
-constexpr int IPC = 8;                     // attention items per workgroup
 constexpr int GRP = 32;                    // 6-value groups of a head group's 192 attention outputs
+
+// How a cell splits its (sequence, KV head) pairs over its workgroups: in whole workgroups (geometry G itself), or
+// end to end on a line of tiles that the workgroups share evenly (EndToEnd<G>).
+template <class G>
+struct EndToEnd : G {};
+template <class G> constexpr bool end_to_end = false;
+template <class G> constexpr bool end_to_end<EndToEnd<G>> = true;
+constexpr int IPW_MAX = 8;                 // attention items per workgroup, at most (end to end)
 
 // Geometry of a cell: PX XCDs, R workgroups, at most NS sequences.
 template <class G, int PX>
@@ -68,27 +75,35 @@ struct CG {
   static constexpr int UQ = (QU + R - 1) / R, UO = (HU + R - 1) / R, UA = (IU + R - 1) / R;  // per workgroup
   static constexpr int TQ = (4 * UQ + 15) / 16, TO = (4 * UO + 15) / 16, TA = (UA + 1) / 2;  // MFMA tiles
   static constexpr int LMROWS = G::V / NWG, TL = LMROWS / 16;
-  static constexpr int TM = TA > 6 ? TA : 6;             // tiles of the LDS reduction (6: IPC items' P.V sums)
+  static constexpr bool E2E = end_to_end<G>;
+  static constexpr int IPC = E2E ? IPW_MAX : 1;          // attention items per workgroup
+  static constexpr int TM = E2E && TA < 6 ? 6 : TA;      // tiles of the LDS reduction (6: the items' P.V sums)
   static constexpr int KSH = G::H / 64, KSI = G::I / 64; // 64-wide k-steps
   static constexpr int XH = G::H + 8, XI = G::I + 8;     // staged row strides (bank spread)
   static constexpr uint32_t NSEG = 2 * PKT;              // ring bytes of a norm weight vector
   static constexpr int LU = (HU + 63) / 64;              // units of an H-vector per lane
   static constexpr int LA = (IU + NCT - 1) / NCT;        // act units per thread and sequence
-  // tokens of a workgroup's attention range: every sequence at the longest context, plus the padding
-  // of short (sequence, head) pairs (1/4 of a workgroup's share each), whole quads of 16-token tiles
-  static constexpr int TILES = NS * G::KVH * ((kMaxSeq + 15) / 16) / R + IPC;
-  static constexpr int SCT = TILES * 16 + IPC * 64;
+  // Most tiles of a workgroup.  Whole workgroups: with T tiles a chunk, n pairs of together N tiles take at most
+  // N / T + n workgroups.  End to end: its share of every sequence at the longest context, plus the padding of
+  // short pairs (1/4 of a share each).  Items start at whole quads of tiles.
+  static constexpr int NP = NS * G::KVH, NT_MAX = NP * ((kMaxSeq + 15) / 16);
+  static constexpr int TILES = E2E ? NT_MAX / R + IPC : (NT_MAX + R - NP - 1) / (R - NP);
+  static constexpr int SCT = E2E ? TILES * 16 + IPC * 64 : (TILES * 16 + 63) / 64 * 64;
+  static_assert(NP < R && NP <= 64, "a workgroup for every pair, a lane for every pair");
+  static_assert(HU >= R && QU >= R && IU >= R, "rows of every projection for each workgroup (the producer divides by them)");
   static_assert(G::H % 64 == 0 && G::I % 64 == 0 && G::H % 4 == 0 && HU <= NCT, "whole k-steps and units");
   static_assert(G::V % (NWG * 16) == 0 && TL % NCW == 0, "LM-head tiles");
   static_assert(G::H * 2 <= int(NSEG) && HU <= NCT, "two packets of norm weights, one unit per thread");
+  static_assert(TM * NCW * 256 >= IPC * NCW * 192 && TO <= TM && TQ <= TM, "the reduction buffer");
   static_assert(TQ <= NCW && NS * LA <= 32, "one QKV tile per wave; pending bits of the act poll");
-  static_assert(R / G::KVH + 2 <= 64, "a (sequence, head) pair has at most 64 chunks");
+  static_assert(R / G::KVH + 2 <= 64, "a lane for every chunk of a pair: a sequence's heads have equally many");
 };
 
 // Exchange region (units of 16 bytes from its base; one layout for both models, so that no unit is
 // read in a format it was not written in): the workgroups' end records per sequence (tag: epoch), the
-// vectors per sequence (tag: epoch, and the layer in the word before it), the attention records keyed
-// by workgroup and item (statistics, 2 units; partial sums, 64 units; tag: (epoch << 5) | layer).
+// vectors per sequence (tag: epoch, and the layer in the word before it; the attention vector: (epoch << 5) |
+// layer), the attention records of each workgroup's items (statistics, 2 units; partial sums, 64 units; the
+// same tag).
 enum CKind { C_X, C_ATT, C_H1, C_QKV, C_ACT };
 template <class G>
 struct CW {
@@ -100,7 +115,7 @@ struct CW {
   static_assert(HU <= 640 && QU <= 640 && IU <= 640, "a vector's lines");
   static constexpr uint32_t REC0 = V0 + LINES * SLOTS * 4;
   static constexpr uint32_t REC = 66;
-  static constexpr uint32_t TOTAL = REC0 + uint32_t(NWG) * IPC * REC;
+  static constexpr uint32_t TOTAL = REC0 + uint32_t(NWG) * IPW_MAX * REC;
   __device__ static uint32_t end(int b, int wg) { return (uint32_t(b) * NWG + uint32_t(wg)) * 16u; }
   // unit u of vector `kind` of sequence slot cs (cell * NS + slot): lane part and uniform part
   __device__ static uint32_t vec_u(int u) { return (V0 + uint32_t(u) / UPL * SLOTS * 4u + uint32_t(u) % UPL) * 16u; }
@@ -108,16 +123,16 @@ struct CW {
   static constexpr uint32_t STRIDE64 = 64 / UPL * SLOTS * 64u;
   __device__ static uint32_t vec_s(int kind, int cs) { return (uint32_t(cs) * 5u + uint32_t(kind)) * 64u; }
   __device__ static uint32_t rec(int wgkey, int k, int unit) {
-    return (REC0 + (uint32_t(wgkey) * IPC + uint32_t(k)) * REC + uint32_t(unit)) * 16u;
+    const uint32_t at = end_to_end<G> ? uint32_t(wgkey) * IPW_MAX + uint32_t(k) : uint32_t(wgkey);
+    return (REC0 + at * REC + uint32_t(unit)) * 16u;
   }
 };
 
-// An attention item: a run of a (sequence, KV head) pair's 16-token tiles.
+// An attention item: a chunk (a run of 16-token tiles) of a (sequence, KV head) pair.
 struct Item {
   int slot, b, g;        // sequence slot in the cell, global sequence, KV head
-  int t0, n;             // first cached token, cached tokens of this run
-  int tile0, ntile;      // first tile in the workgroup's stream, tiles with tokens
-  int quad0;             // running number of its first quad (4 tiles)
+  int t0, n, ntile;      // first cached token, cached tokens and tiles of the chunk
+  int tile0, quad0;      // tiles and quads (of 4 tiles) of the workgroup's items before this one
   int sc0;               // first score slot
   int r0, C, c, k0;      // first workgroup of the pair, its chunks, this one's index, item index in r0
   int leader;            // holds the pair's end: the new token
@@ -126,28 +141,34 @@ struct Item {
 template <class G, int PX>
 struct SmemRest {
   using S = CG<G, PX>;
-  struct Attn {
-    uint16_t q[IPC][5][64];               // roped q heads, new k (leaders), new v (leaders)
-    float wml[IPC][NCW][6];               // per-wave softmax max / sum of the three heads
-    float gml[IPC][6];                    // the pair's max and 1 / sum
-    float snew[IPC][4];                   // leaders: the new token's scores, then its probabilities
-    uint16_t sc[3][S::SCT];               // bf16 scores, then probabilities, per head
+  struct One {
+    float wml[NCW][6];                    // per-wave softmax max / sum of the three heads
+    alignas(16) uint16_t sc[3][S::SCT];   // bf16 scores, then probabilities, per head
   };
+  struct Many {
+    uint16_t q[S::IPC][5][64];            // roped q heads, new k (leaders), new v (leaders)
+    float wml[S::IPC][NCW][6];
+    float gml[S::IPC][6];                 // the pair's max and 1 / sum
+    float snew[S::IPC][4];                // leaders: the new token's scores
+    uint16_t sc[3][S::SCT];
+  };
+  using Attn = std::conditional_t<S::E2E, Many, One>;
   static constexpr int XN = S::NS * S::XI > BMAX * S::XH ? S::NS * S::XI : BMAX * S::XH;
   union {
     alignas(16) uint16_t xs[XN];          // staged activations [sequence][K + 8]
     Attn at;
   };
-  alignas(16) float red[S::TM][NCW][256];  // per-wave MFMA partial tiles; attention: per-wave P.V sums
+  alignas(16) float red[S::TM][NCW][256];  // per-wave MFMA partial tiles; attention: per-wave P.V sums [item][wave][192]
   uint2 res[S::NS][S::UO];                // residual rows of this workgroup (x, then h1)
   float sums[NCW][BMAX];
   LayerW lw[G::L];
   const void* kvp[G::L];
-  Item it[IPC];
-  int32_t blk[S::TILES + IPC];
+  Item it[S::IPC];
+  int32_t blk[S::TILES + S::IPC];
   int32_t sid[BMAX];                      // the cell's sequences by slot
   int32_t cs[BMAX];                       // every sequence's exchange slot
-  int32_t ns, ni, ntile, nquad;
+  int32_t ns, ni, ntile;
+  int32_t slow;                           // a workgroup with the longest chunk (-1: no pair has more than one)
   int32_t sS[BMAX], sPos[BMAX], sId[BMAX];
   long long sSlot[BMAX];
   float lm_val[NCW][BMAX];
@@ -185,10 +206,11 @@ struct PlanC {
 
 // ------------------------------------------------------------------------------------------------
 // Set-up by one wave: the cell's sequences and the workgroup's attention items.
-// Sequences are dealt to the cells in order of falling context length, back and forth.  A cell's
-// (sequence, KV head) pairs lie end to end on a line of 16-token tiles, a short pair padded to a
-// quarter of a workgroup's share (so that a workgroup never holds more than IPC pairs); workgroup r
-// takes tiles [NT r / R, NT (r + 1) / R).
+// Sequences are dealt to the cells in order of falling context length, back and forth.
+// Whole workgroups: a pair of n tiles takes ceil(n / T) workgroups in equal chunks, T the least that all pairs'
+// chunks need no more than R for, and at least TMIN: shorter chunks leave waves idle and widen the pair's exchanges.
+// End to end: the pairs lie on a line of tiles, a short one padded to a quarter of a workgroup's share (so that a
+// workgroup never holds more than IPC pairs); workgroup r takes tiles [NT r / R, NT (r + 1) / R).
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ int wave_scan_incl(int v, int lane) {
 #pragma unroll
@@ -227,43 +249,81 @@ __device__ __forceinline__ void setup(const Params& p, const PlanC<G, PX>& P, Sm
   const int b = on ? *(volatile int*)&sm.sid[slot] : 0;
   const int old = on ? sm.sS[b] - 1 : 0;
   const int tiles = (old + 15) / 16;
-  const int nt0 = __shfl(wave_scan_incl(on ? tiles : 0, lane), 63);
-  const int least = max(1, (nt0 + 4 * S::R - 1) / (4 * S::R));
-  const int nt = on ? max(tiles, least) : 0;
-  const int incl = wave_scan_incl(nt, lane);
-  const int NT = __shfl(incl, 63);
-  const int base = incl - nt;
-  // workgroups that take a share: at least TMIN tiles each while the line is short
-  const int RE = min(S::R, (NT + PK_CELL_TMIN - 1) / PK_CELL_TMIN);
-  auto wg_of = [&](int tile) { return ((tile + 1) * RE - 1) / max(NT, 1); };  // workgroup of a tile of the line
-  const int r0 = wg_of(base), r1 = wg_of(base + max(nt, 1) - 1);
-  int k0 = -1;  // pairs that start at or before r0's first tile
-  const int first = NT > 0 ? split_lo(NT, RE, r0) : 0;
-  for (int j = 0; j < np; ++j) k0 += __shfl(base, j) <= first ? 1 : 0;
-  k0 = lane - k0;
-  const int w0 = P.r < RE ? split_lo(NT, RE, P.r) : NT, w1 = P.r < RE ? split_lo(NT, RE, P.r + 1) : NT;
-  const int a = max(base, w0) - base, e = min(base + nt, w1) - base;  // tiles of the pair in this workgroup
-  const bool have = on && a < e;
-  const uint64_t m = __ballot(have);
-  const int k = __popcll(m & ((uint64_t(1) << lane) - 1u));
-  const int re = min(e, tiles), n = have && re > a ? min(re * 16, old) - a * 16 : 0;
-  const int ntile = (n + 15) / 16, nquad = (ntile + 3) / 4;
-  const int ts = wave_scan_incl(have ? ntile : 0, lane), qs = wave_scan_incl(have ? nquad : 0, lane);
-  if (have && k < IPC) {
-    Item it;
-    it.slot = slot; it.b = b; it.g = g;
-    it.t0 = a * 16; it.n = n;
-    it.tile0 = ts - ntile; it.ntile = ntile;
-    it.quad0 = qs - nquad;
-    it.sc0 = (qs - nquad) * 64;
-    it.r0 = r0; it.C = r1 - r0 + 1; it.c = P.r - r0; it.k0 = k0;
-    it.leader = e == nt;
-    sm.it[k] = it;
-  }
-  if (lane == 63) {
-    sm.ni = min(__popcll(m), IPC);
-    sm.ntile = ts;
-    sm.nquad = qs;
+  if constexpr (S::E2E) {
+    const int nt0 = __shfl(wave_scan_incl(on ? tiles : 0, lane), 63);
+    const int least = max(1, (nt0 + 4 * S::R - 1) / (4 * S::R));
+    const int nt = on ? max(tiles, least) : 0;
+    const int incl = wave_scan_incl(nt, lane);
+    const int NT = __shfl(incl, 63);
+    const int base = incl - nt;
+    // workgroups that take a share: at least TMIN tiles each while the line is short
+    const int RE = min(S::R, (NT + PK_CELL_TMIN - 1) / PK_CELL_TMIN);
+    auto wg_of = [&](int tile) { return ((tile + 1) * RE - 1) / max(NT, 1); };  // workgroup of a tile of the line
+    const int r0 = wg_of(base), r1 = wg_of(base + max(nt, 1) - 1);
+    int k0 = -1;  // pairs that start at or before r0's first tile
+    const int first = NT > 0 ? split_lo(NT, RE, r0) : 0;
+    for (int j = 0; j < np; ++j) k0 += __shfl(base, j) <= first ? 1 : 0;
+    k0 = lane - k0;
+    const int w0 = P.r < RE ? split_lo(NT, RE, P.r) : NT, w1 = P.r < RE ? split_lo(NT, RE, P.r + 1) : NT;
+    const int a = max(base, w0) - base, e = min(base + nt, w1) - base;  // tiles of the pair in this workgroup
+    const bool have = on && a < e;
+    const uint64_t m = __ballot(have);
+    const int k = __popcll(m & ((uint64_t(1) << lane) - 1u));
+    const int re = min(e, tiles), n = have && re > a ? min(re * 16, old) - a * 16 : 0;
+    const int ntile = (n + 15) / 16, nquad = (ntile + 3) / 4;
+    const int ts = wave_scan_incl(have ? ntile : 0, lane), qs = wave_scan_incl(have ? nquad : 0, lane);
+    if (have && k < S::IPC) {
+      Item it;
+      it.slot = slot; it.b = b; it.g = g;
+      it.t0 = a * 16; it.n = n;
+      it.tile0 = ts - ntile; it.ntile = ntile;
+      it.quad0 = qs - nquad;
+      it.sc0 = (qs - nquad) * 64;
+      it.r0 = r0; it.C = r1 - r0 + 1; it.c = P.r - r0; it.k0 = k0;
+      it.leader = e == nt;
+      sm.it[k] = it;
+    }
+    if (lane == 63) {
+      sm.ni = min(__popcll(m), S::IPC);
+      sm.ntile = ts;
+    }
+  } else {
+    const int nt = on ? max(tiles, 1) : 0;
+    const int NT = __shfl(wave_scan_incl(nt, lane), 63);
+    int t = max(PK_CELL_TMIN, (NT + S::R - 1) / S::R);
+    for (int hi = max(t, (NT + S::R - np - 1) / (S::R - np)); t < hi;) {  // hi is always enough
+      const int mid = (t + hi) / 2;
+      float s[1] = {float((nt + mid - 1) / mid)};
+      wave_sum_n<1>(s);
+      if (s[0] <= float(S::R)) hi = mid;
+      else t = mid + 1;
+    }
+    const int C = (nt + t - 1) / t;
+    const int r0 = wave_scan_incl(C, lane) - C, c = P.r - r0;
+    const bool have = on && c >= 0 && c < C;  // in one lane at most
+    if (have) {
+      const int a = nt * c / C, e = min(nt * (c + 1) / C, tiles);
+      Item it;
+      it.slot = slot; it.b = b; it.g = g;
+      it.t0 = a * 16;
+      it.n = e > a ? min(e * 16, old) - a * 16 : 0;
+      it.tile0 = 0; it.ntile = max(e - a, 0); it.quad0 = 0; it.sc0 = 0;
+      it.r0 = r0; it.C = C; it.c = c; it.k0 = 0;
+      it.leader = c == C - 1;
+      sm.it[0] = it;
+      sm.ntile = it.ntile;
+    }
+    const uint64_t m = __ballot(have);
+    float longest[1] = {on && C > 1 ? float((nt + C - 1) / C) : 0.f};
+    const float mine = longest[0];
+    wave_max_n<1>(longest);
+    const uint64_t sl = __ballot(mine > 0.f && mine == longest[0]);
+    const int slow = sl ? __shfl(r0 + C - 1, __ffsll((unsigned long long)sl) - 1) : -1;
+    if (lane == 0) {
+      sm.ni = m ? 1 : 0;
+      if (!m) sm.ntile = 0;
+      sm.slow = slow;
+    }
   }
 }
 
@@ -348,7 +408,7 @@ __device__ __forceinline__ void producer(const Params& p, const PlanC<G, PX>& P,
   const uint32_t vho = lo * hb + col, vio = lo * ib + col;
   // gate/up: 4 gate rows, then the up rows of the same act unit
   const uint32_t vg = uint32_t(prow < 4 ? prow : G::I + prow - 4) * hb + col;
-  const int ntile = __builtin_amdgcn_readfirstlane(sm.ntile);
+  const int ntile = __builtin_amdgcn_readfirstlane(sm.ntile), ni = __builtin_amdgcn_readfirstlane(sm.ni);
   constexpr int BV = (S::TILES + 63) / 64;
   int blkv[BV];  // lane i: block ids of tiles i, i + 64, ...
 #pragma unroll
@@ -363,12 +423,12 @@ __device__ __forceinline__ void producer(const Params& p, const PlanC<G, PX>& P,
       room(gn);
       if (dead) break;
       const int tile = int(i >> 1);
-      while (tile >= end) {
-        ++k;
-        tile0 = __builtin_amdgcn_readfirstlane(sm.it[k].tile0);
-        end = tile0 + __builtin_amdgcn_readfirstlane(sm.it[k].ntile);
-        last = __builtin_amdgcn_readfirstlane(sm.it[k].n) - 1;
-        head = (long long)__builtin_amdgcn_readfirstlane(sm.it[k].g) * p.head_stride + off;
+      while (tile >= end && k + 1 < ni) {
+        const Item& it = sm.it[++k];
+        tile0 = __builtin_amdgcn_readfirstlane(it.tile0);
+        end = tile0 + __builtin_amdgcn_readfirstlane(it.ntile);
+        last = __builtin_amdgcn_readfirstlane(it.n) - 1;
+        head = (long long)__builtin_amdgcn_readfirstlane(it.g) * p.head_stride + off;
       }
       int blk = 0;
 #pragma unroll
@@ -482,6 +542,13 @@ struct CC {
   }
   __device__ __forceinline__ uint4 ring16(uint32_t at, uint32_t lo) const {
     return *reinterpret_cast<const uint4*>(sm.ring + ring_at(at, lo));
+  }
+  // ds_read_b64_tr_b16: of 16 lanes, lane 4 j + q gives the address of 4 values, lane i gets value i % 4 of lanes i / 4,
+  // 4 + i / 4, 8 + i / 4 and 12 + i / 4
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  __device__ __forceinline__ uint2 ring_tr(uint32_t at, uint32_t lo) const {
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(sm.ring + ring_at(at, lo))));
   }
   __device__ __forceinline__ uint2 ring8(uint32_t at, uint32_t lo) const {
     return *reinterpret_cast<const uint2*>(sm.ring + ring_at(at, lo));
@@ -659,6 +726,16 @@ __device__ __forceinline__ void stage_att_n(CC<G, PX>& C, int l) {
   u32x4 x[N];
   constexpr int AU = G::H / 6;
   const uint32_t o = CW<G>::vec_u(min(C.ct, AU - 1)), tg = C.tag(l);
+  if constexpr (!S::E2E && S::NS > 4) {
+    // Workgroups with short chunks wait here while others still stream: for one unit, a sum of the longest
+    // chunk (the vectors follow it by an exchange), instead of up to 20 KB a try
+    const int slow = __builtin_amdgcn_readfirstlane(C.sm.slow);
+    if (slow >= 0) {
+      u32x4 y[1];
+      const uint32_t os = CW<G>::rec(C.P.cell * S::R + slow, 0, 2);
+      C.template poll<1>(55, 1u, [&](const u32x4& u) { return u.w == tg; }, [&](int) { return os; }, [&](int) { return 0u; }, y);
+    }
+  }
   C.template poll<N>(44 + C_ATT, (1u << C.ns) - 1u, [&](const u32x4& u) { return u.w == tg; }, [&](int) { return o; },
                      [&](int i) { return CW<G>::vec_s(C_ATT, C.slot0() + i); }, x);
   if (C.ct < AU)
@@ -848,10 +925,300 @@ __device__ __forceinline__ floatx4 red_sum(const CC<G, PX>& C, int t, int lane) 
 }
 
 // ------------------------------------------------------------------------------------------------
-// Attention over this workgroup's items.
+// Attention over this workgroup's one chunk (of four waves, two barriers).
 // ------------------------------------------------------------------------------------------------
 template <class G, int PX>
-__device__ __forceinline__ void attention(CC<G, PX>& C, int l) {
+__device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
+  using S = CG<G, PX>;
+  using W = CW<G>;
+  const Params& p = C.p;
+  SmemC<G, PX>& sm = C.sm;
+  const int lane = C.lane, w = C.cw;
+  auto tr = [&](int ev) { if (C.ct == 0) trace_at(p, l, ev, p.n_layers); };
+  auto one = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+  if (one(sm.ni) == 0) return;
+  const Item& it = sm.it[0];
+  const int g = one(it.g), n = one(it.n), nt = one(it.ntile), Cc = one(it.C), ci = one(it.c);
+  const int r0 = C.P.cell * S::R + one(it.r0);  // record key of the pair's first chunk
+  const int slot = C.slot0() + one(it.slot);
+  const int nquad = (nt + 3) / 4;
+  const int me = C.P.cell * S::R + C.P.r;
+  const uint32_t tg = C.tag(l);
+  const uint32_t kpos = C.pos, vpos = kpos + uint32_t(nt) * 2u * PKT;
+  C.pos = vpos + uint32_t(nt) * 2u * PKT;
+  const bool has_new = w == NCW - 1 && one(it.leader);  // the new token is wave 3's, in the chunk with the pair's end
+  // ---- q straight into MFMA operands: lane (head lane % 4, piece j = lane / 16) takes dims 8j .. 8j + 7 and 32 + 8j
+  // .. of its head, which are the two halves of four units (two RoPE pairs each) of one 64-byte line; the new
+  // token's k alike, for every column of an operand, and v unit lane / 4 (4 dims): one round trip ----
+  const int hr = (lane & 3) < 3 ? (lane & 3) : 0, pj = lane >> 4;
+  static_assert(W::UPL == 4, "a lane's four units share a line");
+  u32x4 x[9];
+  {
+    const uint32_t oq = W::vec_u(g * 48 + hr * 16 + 4 * pj), ok = W::vec_u((G::NH + g) * 16 + 4 * pj);
+    const uint32_t ov = W::vec_u((G::NH + G::KVH + g) * 16 + (lane >> 2)), sq = W::vec_s(C_QKV, slot);
+    C.template poll<9>(50, has_new ? 0x1ffu : 0xfu, [&](const u32x4& u) { return C.vec_ok(u, l); },
+                       [&](int i) { return i < 8 ? (i < 4 ? oq : ok) + 16u * uint32_t(i % 4) : ov; }, [&](int) { return sq; }, x);
+  }
+  auto half = [&](int i, int h) {
+    return h == 0 ? make_uint4(x[i].x, x[i + 1].x, x[i + 2].x, x[i + 3].x)
+                  : make_uint4(x[i].y, x[i + 1].y, x[i + 2].y, x[i + 3].y);
+  };
+  const uint4 k0 = half(4, 0), k1 = half(4, 1);
+  const uint2 vnew = make_uint2(x[8].x, x[8].y);
+  tr(4);
+  float vn[3] = {-INFINITY, -INFINITY, -INFINITY};
+  const bf16x8 qa0 = __builtin_bit_cast(bf16x8, half(0, 0)), qa1 = __builtin_bit_cast(bf16x8, half(0, 1));
+  // ---- scores: quads of 4 tiles (64 tokens), dealt round-robin to the waves.  D = Q K^T on the matrix
+  // cores with the three q heads in rows 4i .. 4i + 2 of every row block i, so lane l takes its token's
+  // three scores from tile l / 16's accumulator: token l of the quad ----
+  float m[3] = {-INFINITY, -INFINITY, -INFINITY};
+  uint16_t* sc = &sm.at.sc[0][lane];
+  for (int j = w; j < nquad; j += NCW) {
+    const int tl = min(4, nt - 4 * j);
+    const uint32_t at = kpos + uint32_t(4 * j) * 2u * PKT;
+    C.release(at);
+    C.wait_filled(at + uint32_t(tl) * 2u * PKT);
+    const uint32_t lo = uint32_t((lane & 15) >> 3) * PKT + uint32_t(lane & 7) * 128u;
+    uint4 ka[4][2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        ka[t][h] = C.ring16(at + uint32_t(min(t, tl - 1)) * 2u * PKT, lo + uint32_t((4 * h + pj + (lane & 7)) & 7) * 16u);
+    floatx4 d[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      d[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa0, __builtin_bit_cast(bf16x8, ka[t][0]),
+                                                    floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      d[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa1, __builtin_bit_cast(bf16x8, ka[t][1]), d[t], 0, 0, 0);
+    const bool in = j * 64 + lane < n;
+#pragma unroll
+    for (int h = 0; h < 3; ++h) {
+      const float y = lane < 32 ? (lane < 16 ? d[0][h] : d[1][h]) : (lane < 48 ? d[2][h] : d[3][h]);
+      const float v = in ? rnd(y) * 0.125f : -INFINITY;  // bf16(q.k) / 8 (HF)
+      sc[h * S::SCT + j * 64] = uint16_t(f2bf(v));
+      m[h] = fmaxf(m[h], v);
+    }
+  }
+  if (has_new) {
+    floatx4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa0, __builtin_bit_cast(bf16x8, k0), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa1, __builtin_bit_cast(bf16x8, k1), d, 0, 0, 0);
+#pragma unroll
+    for (int h = 0; h < 3; ++h) {
+      vn[h] = rnd(d[h]) * 0.125f;
+      m[h] = fmaxf(m[h], vn[h]);
+    }
+  }
+  // ---- the wave's statistics ----
+  wave_max_n<3>(m);
+  float ls[3] = {0.f, 0.f, 0.f};
+  wait_lgkm0();
+  for (int j = w; j < nquad; j += NCW)
+#pragma unroll
+    for (int h = 0; h < 3; ++h) {
+      const float v = bf2f(sc[h * S::SCT + j * 64]);
+      ls[h] += v == -INFINITY ? 0.f : __expf(v - m[h]);
+    }
+  wave_sum_n<3>(ls);
+  if (has_new)
+#pragma unroll
+    for (int h = 0; h < 3; ++h) ls[h] += __expf(vn[h] - m[h]);
+  if (lane < 6) {
+    const int h = lane < 3 ? lane : lane - 3;
+    const float a = h == 0 ? m[0] : h == 1 ? m[1] : m[2], b = h == 0 ? ls[0] : h == 1 ? ls[1] : ls[2];
+    sm.at.wml[w][lane] = lane < 3 ? a : b;
+  }
+  C.release(vpos);
+  C.cbar();
+  // ---- the chunk's statistics: the waves' merged by every wave (lanes 0-11: wave lane % 4, head lane / 4) and
+  // published by wave 0 where the pair has other chunks; then the pair's (lane i: chunk i) ----
+  auto rl = [](float v, int i) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i));
+  };
+  float M[3], inv[3];
+  {
+    float mq = -INFINITY, lq = 0.f;
+    if (lane < 12) { mq = sm.at.wml[lane & 3][lane >> 2]; lq = sm.at.wml[lane & 3][3 + (lane >> 2)]; }
+    float mx = fmaxf(mq, dpp<0xb1>(mq, mq));
+    mx = fmaxf(mx, dpp<0x4e>(mx, mx));
+    float ex = mq == -INFINITY ? 0.f : lq * __expf(mq - mx);
+    ex += dpp<0xb1>(0.f, ex);
+    ex += dpp<0x4e>(0.f, ex);
+#pragma unroll
+    for (int h = 0; h < 3; ++h) { M[h] = rl(mx, 4 * h); inv[h] = rl(ex, 4 * h); }
+  }
+  if (Cc > 1) {
+    if (w == 0) {
+      skew_delay(p.skew, C.P.wg, l, 14);
+      if (lane < 2)
+        C.st(W::rec(me, 0, lane),
+             lane == 0 ? u32x4{__float_as_uint(M[0]), __float_as_uint(M[1]), __float_as_uint(M[2]), tg}
+                       : u32x4{__float_as_uint(inv[0]), __float_as_uint(inv[1]), __float_as_uint(inv[2]), tg});
+    }
+    tr(5);
+    u32x4 y[2];
+    const uint32_t o = W::rec(r0 + min(lane, Cc - 1), 0, 0);
+    C.template poll<2>(51, 3u, [&](const u32x4& u) { return u.w == tg; }, [&](int i) { return o + 16u * uint32_t(i); },
+                       [&](int) { return 0u; }, y);
+    const bool mine = lane < Cc;
+    float mk[3];
+#pragma unroll
+    for (int h = 0; h < 3; ++h) M[h] = mk[h] = mine ? __uint_as_float(h == 0 ? y[0].x : h == 1 ? y[0].y : y[0].z) : -INFINITY;
+    wave_max_n<3>(M);
+#pragma unroll
+    for (int h = 0; h < 3; ++h) {
+      const float lk = __uint_as_float(h == 0 ? y[1].x : h == 1 ? y[1].y : y[1].z);
+      inv[h] = mk[h] == -INFINITY ? 0.f : lk * __expf(mk[h] - M[h]);
+    }
+    wave_sum_n<3>(inv);
+  }
+  // ---- KV append of the new token (block360_kernel.inc:124-135), where no load follows for 1 us and more
+  // (a wave's loads wait for its earlier stores): k unit u
+  // (k0, k1 word u % 4 of piece u / 4) holds dims 2u, 2u + 1 and 32 + 2u, 33 + 2u, v unit u dims 4u .. 4u + 3 ----
+  if (has_new) {
+    const long long ns = sm.sSlot[one(it.b)];
+    if (ns >= 0) {
+      uint16_t* cache = reinterpret_cast<uint16_t*>(const_cast<void*>(sm.kvp[l]));
+      const long long e = (ns / 16) * p.block_stride + (ns % 16) * p.token_stride + (long long)g * p.head_stride;
+      uint16_t *kd = cache + e + p.k_off + 8 * pj, *vd = cache + e + p.v_off + lane;  // v: lanes 0, 4, ...
+      if (((reinterpret_cast<uintptr_t>(kd) | reinterpret_cast<uintptr_t>(vd - lane)) & 15u) == 0) {
+        if ((lane & 15) == 0) {
+          st_global16(kd, k0.x, k0.y, k0.z, k0.w);
+          st_global16(kd + 32, k1.x, k1.y, k1.z, k1.w);
+        }
+        typedef __attribute__((address_space(1))) uint64_t g_u64;
+        if ((lane & 3) == 0) *(g_u64*)(vd) = uint64_t(vnew.x) | (uint64_t(vnew.y) << 32);
+      } else {
+        const uint32_t a[4] = {k0.x, k0.y, k0.z, k0.w}, b[4] = {k1.x, k1.y, k1.z, k1.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if ((lane & 15) == 0) {
+            st_global2(kd + 2 * i, uint16_t(a[i] & 0xffffu));
+            st_global2(kd + 2 * i + 1, uint16_t(a[i] >> 16));
+            st_global2(kd + 32 + 2 * i, uint16_t(b[i] & 0xffffu));
+            st_global2(kd + 32 + 2 * i + 1, uint16_t(b[i] >> 16));
+          }
+        if ((lane & 3) == 0) {
+          st_global2(vd, uint16_t(vnew.x & 0xffffu));
+          st_global2(vd + 1, uint16_t(vnew.x >> 16));
+          st_global2(vd + 2, uint16_t(vnew.y & 0xffffu));
+          st_global2(vd + 3, uint16_t(vnew.y >> 16));
+        }
+      }
+    }
+  }
+  tr(6);
+  // ---- p = bf16(exp(s - M) / L) with the pair's M and L (HF); P.V on the matrix cores, p of the heads in the
+  // rows as q above, 32 tokens a step: lane l's tokens are packet l / 16 of the step's four, its dims l % 16 of each
+  // block of 16.  A lane's eight tokens of one dim come from two transposing reads, four lanes to a row's 32 bytes.
+  // (In fp32 dot products on the vector unit this took 0.84 us a quad.) ----
+  float* wo = &sm.red[0][0][0];  // [wave][192]
+  const int tr_row = (lane & 15) >> 2;
+#pragma unroll
+  for (int h = 0; h < 3; ++h) inv[h] = 1.0f / inv[h];
+  floatx4 acc[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) acc[d] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int j = w; j < nquad; j += NCW) {
+    const int tl = min(4, nt - 4 * j);
+    const uint32_t at = vpos + uint32_t(4 * j) * 2u * PKT;
+    C.release(at);
+    uint16_t* pq = &sm.at.sc[0][j * 64];
+#pragma unroll
+    for (int h = 0; h < 3; ++h) {
+      uint16_t* s = pq + h * S::SCT + lane;
+      *s = uint16_t(f2bf(__expf(bf2f(*s) - M[h]) * inv[h]));
+    }
+    C.wait_filled(at + uint32_t(tl) * 2u * PKT);
+    wait_lgkm0();
+    asm volatile("" ::: "memory");  // the operands read below are these stores, of another type
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {  // tiles past the run read its last one again, with probability 0
+      const uint4 pa = *reinterpret_cast<const uint4*>(pq + hr * S::SCT + 32 * i + 8 * pj);
+      uint4 vb[4];
+      const uint32_t pk = uint32_t(2 * min(2 * i + (pj >> 1), tl - 1) + (pj & 1)) * PKT + uint32_t(lane & 1) * 8u;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const int c = 2 * d + ((lane >> 1) & 1);  // 16-byte piece of the row
+        const uint2 lo = C.ring_tr(at, pk + uint32_t(tr_row) * 128u + uint32_t((c + tr_row) & 7) * 16u);
+        const uint2 hi = C.ring_tr(at, pk + uint32_t(tr_row + 4) * 128u + uint32_t((c + tr_row + 4) & 7) * 16u);
+        vb[d] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+      }
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+        acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pa), __builtin_bit_cast(bf16x8, vb[d]),
+                                                        acc[d], 0, 0, 0);
+    }
+  }
+  const float vf = (lane & 1) ? bf_hi((lane & 2) ? vnew.y : vnew.x) : bf_lo((lane & 2) ? vnew.y : vnew.x);
+#pragma unroll
+  for (int h = 0; h < 3; ++h) {  // lane: dim
+    float v = lane < 32 ? (lane < 16 ? acc[0][h] : acc[1][h]) : (lane < 48 ? acc[2][h] : acc[3][h]);
+    if (has_new) v = fmaf(rnd(__expf(vn[h] - M[h]) * inv[h]), vf, v);
+    wo[w * 192 + h * 64 + lane] = v;
+  }
+  C.release(C.pos);
+  C.cbar();
+  // ---- publish (wave 0): a pair in one chunk gives its attention values, others their fp32 partial sums ----
+  const uint32_t att = W::vec_s(C_ATT, slot);
+  if (w == 0) {
+    skew_delay(p.skew, C.P.wg, l, 15);
+    if (Cc > 1) {
+      float v[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        v[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < NCW; ++j) v[i] += wo[j * 192 + 3 * lane + i];
+      }
+      C.st(W::rec(me, 0, 2 + lane), u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), tg});
+    } else if (lane < GRP) {
+      float v[6];
+#pragma unroll
+      for (int i = 0; i < 6; ++i) {
+        v[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < NCW; ++j) v[i] += wo[j * 192 + 6 * lane + i];
+      }
+      C.st(W::vec_u(g * GRP + lane), u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), tg}, att);
+    }
+    tr(7);
+  }
+  // ---- combine (wave 2): chunk c of a pair adds groups [32 c / C, 32 (c + 1) / C) of 6 values over the C chunks, in
+  // chunk order, two lanes a group, and publishes them ----
+  const int g0 = GRP * ci / Cc, ng = GRP * (ci + 1) / Cc - g0;
+  if (w == 2 && Cc > 1 && ng > 0) {
+    const uint32_t ou = uint32_t(2 + 2 * g0 + min(lane, 2 * ng - 1)) * 16u;
+    float v[3] = {0.f, 0.f, 0.f};
+    constexpr int N = 13;  // a sequence alone in its cell has up to 25 chunks a head
+    for (int c0 = 0; c0 < Cc; c0 += N) {
+      u32x4 y[N];
+      const int nc = min(N, Cc - c0);
+      C.template poll<N>(52, (1u << nc) - 1u, [&](const u32x4& u) { return u.w == tg; }, [&](int) { return ou; },
+                         [&](int i) { return W::rec(r0 + c0 + i, 0, 0); }, y);
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (i < nc) {
+          v[0] += __uint_as_float(y[i].x);
+          v[1] += __uint_as_float(y[i].y);
+          v[2] += __uint_as_float(y[i].z);
+        }
+    }
+    float y[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) y[i] = dpp<0xb1>(0.f, v[i]);  // the pair's other lane
+    if ((lane & 1) == 0 && lane < 2 * ng)
+      C.st(W::vec_u(g * GRP + g0 + (lane >> 1)), u32x4{pack2(v[0], v[1]), pack2(v[2], y[0]), pack2(y[1], y[2]), tg}, att);
+  }
+  tr(8);
+}
+// ------------------------------------------------------------------------------------------------
+// Attention over this workgroup's items, end to end.
+// ------------------------------------------------------------------------------------------------
+template <class G, int PX>
+__device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
   using S = CG<G, PX>;
   using W = CW<G>;
   const Params& p = C.p;
@@ -1268,7 +1635,8 @@ __device__ __forceinline__ void consumer(const Params& p, const PlanC<G, PX>& P,
     tr(l, 3);
     // ---------------- attention ----------------
     C.refresh();
-    attention<G, PX>(C, l);
+    if constexpr (S::E2E) attention_many<G, PX>(C, l);
+    else attention_one<G, PX>(C, l);
     // ---------------- O + residual ----------------
     C.refresh();
     auto rows_out = [&](int kind, int site, bool outputs) {
@@ -1541,9 +1909,25 @@ static int launch(const Params& p, const void* region, hipStream_t stream, int c
 // make every exchange wider.  us per step at 1 / 2 / 4 XCDs (and the kernel of one cell of eight,
 // decode_kernel_b): 360M batch 4, contexts 100..2000: 1,893 / 926 / 759 (1,365); batch 16, 1000..4000:
 // 2,291 / 1,200 / 1,167 (1,771); 135M batch 4: 684 / 596 / 624 (1,055); batch 16: 807 / 737 / 829 (1,342).
+//
+// Pairs in whole workgroups while the block tables' capacity is moderate, end to end above.  One chunk a workgroup takes
+// two barriers and no staging of q and k, and P.V runs on the matrix cores; but rounded up to whole workgroups
+// the longest chunk is 4 % (4 sequences) to 20 % (16) longer than an even share, which counts once the stream of
+// K and V bounds the step.  us per step end to end / whole: 360M batch 3, 100..2000: 728 / 693; batch 4, 40..60: 760 / 576,
+// 9000..12000: 993 / 985; batch 8, 100..2000: 818 / 787, 1000..4000: 860 / 833, 3000..9000: 1,106 / 1,119; batch 12,
+// 1000..4000: 996 / 992, 3000..9000: 1,446 / 1,474; batch 16, 40..60: 978 / 781, 100..2000: 1,003 / 956, 1000..4000:
+// 1,161 / 1,160, 8000..12000: 2,404 / 2,773; 135M batch 7, 100..2000: 620 / 588; batch 16, 100..2000: 653 / 635,
+// 3000..9000: 973 / 1,059.  (The second and later items of a workgroup in the one-chunk form: slower than
+// either, 1,800 us at batch 16, 3000..9000.)
+constexpr long long kWholeTokens = 61440;
+template <class G, int PX>
+static int cell_launch_one(const Params& p, const void* region, hipStream_t stream, int cooperative) {
+  if ((long long)p.B * p.max_seq <= kWholeTokens) return cell::launch<G, PX>(p, region, stream, cooperative);
+  return cell::launch<cell::EndToEnd<G>, PX>(p, region, stream, cooperative);
+}
 int cell_launch(int model, const Params& p, const void* region, hipStream_t stream, int cooperative) {
-  if (model == PK_MODEL_SMOLLM2_360M) return cell::launch<G360, 4>(p, region, stream, cooperative);
-  if (model == PK_MODEL_SMOLLM2_135M) return cell::launch<G135, 2>(p, region, stream, cooperative);
+  if (model == PK_MODEL_SMOLLM2_360M) return cell_launch_one<G360, 4>(p, region, stream, cooperative);
+  if (model == PK_MODEL_SMOLLM2_135M) return cell_launch_one<G135, 2>(p, region, stream, cooperative);
   return PK_ERR_MODEL;
 }
 size_t cell_region_bytes() {

@@ -69,3 +69,26 @@ def test_other_cache_strides_give_the_same_bits():
         assert torch.equal(k1[key], k2[key]), key
     for a, b in zip(after, case.kvd):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("base", [O.SMOLLM2_360M, O.SMOLLM2_135M], ids=["360m", "135m"])
+@pytest.mark.parametrize("capacity", [6816, 6832], ids=["whole_workgroups", "end_to_end"])
+def test_both_splits_of_the_pairs_against_oracle(capacity, base):
+    """The same nine sequences at the last block table capacity of the one split and the first of the other
+    (9 * 6,816 <= 61,440 < 9 * 6,832): chunks of one tile, of a quad and one token more, pairs without a
+    cached token."""
+    _need_gpu()
+    contexts = [5, 300, 41, 1025, 257, 1, 258, 17, 2100]
+    case = GC.random_kv_case(O.with_layers(base, 2), 441, contexts, capacity=capacity)
+    ids, pos = [7 + 5 * b for b in range(9)], [S - 1 for S in contexts]
+    got, want = case.kernel_step(ids, pos), case.oracle_step(ids, pos)
+    # Two layers of either end at most 1.0 % (relative norm of the logits) from the step in 64 bits, so two
+    # right results at most 2.0 % from each other
+    for b in range(9):
+        d, r = got["logits"][b].float().cpu(), want["logits"][b].float().cpu()
+        assert (d - r).norm() <= 0.02 * r.norm(), (capacity, b, ((d - r).norm() / r.norm()).item())
+    for li in range(2):
+        for b, S in enumerate(contexts):
+            slot = case.kv.slot(b, S - 1)
+            new = case.kvd[li][slot // 16, :, slot % 16].cpu().float()
+            assert torch.allclose(new, case.kv.caches[li][slot // 16, :, slot % 16].float(), rtol=2 ** -6, atol=2e-2), (li, b)
