@@ -1,4 +1,4 @@
-// SmolLM2 batched decode step (3..16 sequences) on cells of XCDs, one persistent kernel per step for
+// SmolLM2-135M batched decode step (3..16 sequences) on cells of XCDs, one persistent kernel per step for
 // gfx950 (MI355X).
 //
 // The 8 XCDs are grouped into cells of PX neighbouring XCDs (workgroup wg runs on XCD wg % 8 under
@@ -99,7 +99,7 @@ struct CG {
   static_assert(R / G::KVH + 2 <= 64, "a lane for every chunk of a pair: a sequence's heads have equally many");
 };
 
-// Exchange region (units of 16 bytes from its base; one layout for both models, so that no unit is
+// Exchange region (units of 16 bytes from its base; one layout for both splits of the pairs, so that no unit is
 // read in a format it was not written in): the workgroups' end records per sequence (tag: epoch), the
 // vectors per sequence (tag: epoch, and the layer in the word before it; the attention vector: (epoch << 5) |
 // layer), the attention records of each workgroup's items (statistics, 2 units; partial sums, 64 units; the
@@ -1905,34 +1905,22 @@ static int launch(const Params& p, const void* region, hipStream_t stream, int c
 
 }  // namespace cell
 
-// Cells of four XCDs for 360M, of two for 135M: fewer XCDs a cell read the weights more often, more XCDs
-// make every exchange wider.  us per step at 1 / 2 / 4 XCDs (and the kernel of one cell of eight,
-// decode_kernel_b): 360M batch 4, contexts 100..2000: 1,893 / 926 / 759 (1,365); batch 16, 1000..4000:
-// 2,291 / 1,200 / 1,167 (1,771); 135M batch 4: 684 / 596 / 624 (1,055); batch 16: 807 / 737 / 829 (1,342).
+// Cells of two XCDs: fewer XCDs a cell read the weights more often, more XCDs make every exchange wider.  us per
+// step at 1 / 2 / 4 XCDs (and the kernel of one cell of eight, decode_kernel_b): batch 4: 684 / 596 / 624 (1,055);
+// batch 16: 807 / 737 / 829 (1,342).
 //
 // Pairs in whole workgroups while the block tables' capacity is moderate, end to end above.  One chunk a workgroup takes
 // two barriers and no staging of q and k, and P.V runs on the matrix cores; but rounded up to whole workgroups
-// the longest chunk is 4 % (4 sequences) to 20 % (16) longer than an even share, which counts once the stream of
-// K and V bounds the step.  us per step end to end / whole: 360M batch 3, 100..2000: 728 / 693; batch 4, 40..60: 760 / 576,
-// 9000..12000: 993 / 985; batch 8, 100..2000: 818 / 787, 1000..4000: 860 / 833, 3000..9000: 1,106 / 1,119; batch 12,
-// 1000..4000: 996 / 992, 3000..9000: 1,446 / 1,474; batch 16, 40..60: 978 / 781, 100..2000: 1,003 / 956, 1000..4000:
-// 1,161 / 1,160, 8000..12000: 2,404 / 2,773; 135M batch 7, 100..2000: 620 / 588; batch 16, 100..2000: 653 / 635,
-// 3000..9000: 973 / 1,059.  (The second and later items of a workgroup in the one-chunk form: slower than
-// either, 1,800 us at batch 16, 3000..9000.)
+// the longest chunk is longer than an even share (20 % at 16 sequences), which counts once the stream of
+// K and V bounds the step.  us per step end to end / whole: batch 7, 100..2000: 620 / 588; batch 16, 100..2000: 653 /
+// 635, 3000..9000: 973 / 1,059.  (The second and later items of a workgroup in the one-chunk form: slower than
+// either.)
 constexpr long long kWholeTokens = 61440;
-template <class G, int PX>
-static int cell_launch_one(const Params& p, const void* region, hipStream_t stream, int cooperative) {
-  if ((long long)p.B * p.max_seq <= kWholeTokens) return cell::launch<G, PX>(p, region, stream, cooperative);
-  return cell::launch<cell::EndToEnd<G>, PX>(p, region, stream, cooperative);
+constexpr int kPX = 2;
+int cell_launch(const Params& p, const void* region, hipStream_t stream, int cooperative) {
+  if ((long long)p.B * p.max_seq <= kWholeTokens) return cell::launch<G135, kPX>(p, region, stream, cooperative);
+  return cell::launch<cell::EndToEnd<G135>, kPX>(p, region, stream, cooperative);
 }
-int cell_launch(int model, const Params& p, const void* region, hipStream_t stream, int cooperative) {
-  if (model == PK_MODEL_SMOLLM2_360M) return cell_launch_one<G360, 4>(p, region, stream, cooperative);
-  if (model == PK_MODEL_SMOLLM2_135M) return cell_launch_one<G135, 2>(p, region, stream, cooperative);
-  return PK_ERR_MODEL;
-}
-size_t cell_region_bytes() {
-  static_assert(cell::CW<G360>::TOTAL == cell::CW<G135>::TOTAL, "one layout");
-  return size_t(cell::CW<G360>::TOTAL) * 16;
-}
+size_t cell_region_bytes() { return size_t(cell::CW<G135>::TOTAL) * 16; }
 
 }  // namespace pk

@@ -1,7 +1,6 @@
 // SmolLM2 single-token decode step as one persistent HIP kernel per step for gfx950 (MI355X): the
-// general batch-1 kernel (decode_kernel) and the batched kernel of two sequences with per-layer outputs
-// or stage capture, and of given hidden states (decode_kernel_b); the split-role batch-1 kernel is in
-// decode_sr.hip, the kernel of three or more sequences in decode_cell.hip.  The launch is an ordinary hipLaunchKernel of one workgroup
+// general batch-1 kernel (decode_kernel) and the batched kernel (decode_kernel_b); the split-role batch-1
+// kernel is in decode_sr.hip, 135M's kernel of three or more sequences in decode_cell.hip.  The launch is an ordinary hipLaunchKernel of one workgroup
 // per CU, which relies on all 256 workgroups being resident at once (true on an otherwise idle
 // device: a workgroup waiting for one that is not resident gives up after its bounded wait and the
 // step comes back poisoned and reported); PK_LAUNCH=cooperative or pk_set_option(PK_OPT_COOPERATIVE)
@@ -3603,11 +3602,14 @@ static int decode_impl(void* stream, int B, int n_layers, const void* input_ids,
         }
         return PK_OK;
       }
-      // three or more: cells of XCDs, each decoding its own sequences (360M, three sequences of 100..2000
-      // tokens: 748 us against 1,329 here); two with layer_outputs and given hidden states stay here
-      if (B > 2 && !input_hidden)
-        return cell_launch(G::H == 960 ? PK_MODEL_SMOLLM2_360M : PK_MODEL_SMOLLM2_135M, p,
-                           reinterpret_cast<const uint8_t*>(state->ws) + cell_region_off(), s, opt_cooperative());
+      // 135M, three or more: cells of XCDs, each decoding its own sequences (seven sequences of 100..2000 tokens:
+      // 588 us against 1,191 here).  The cells sum in another order, and one rounding that falls the other way
+      // travels through the layers: the logits of the two kernels, both as far from 64-bit arithmetic, are 0.017 to
+      // 0.026 apart (relative norm, six seeds) for 135M and 0.022 to 0.038 for 360M.  More than 0.03 is not taken for
+      // speed, so 360M stays here (four sequences: 1,388 us, 731 on cells; sixteen: 1,644 and 1,106).
+      if constexpr (G::H == 576)
+        if (B > 2 && !input_hidden)
+          return cell_launch(p, reinterpret_cast<const uint8_t*>(state->ws) + cell_region_off(), s, opt_cooperative());
       return launch<G, true>(p, s);
     }
   return batch1(p);

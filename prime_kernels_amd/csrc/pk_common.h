@@ -163,8 +163,8 @@ __attribute__((visibility("hidden"))) size_t sr_local_bytes(int wide);
 __attribute__((visibility("hidden"))) int sr_max_seq(int model, int wide);
 
 // Batched kernel on cells of XCDs (decode_cell.hip): launch, and the bytes of its exchange region.
-__attribute__((visibility("hidden"))) int cell_launch(int model, const Params& p, const void* region,
-                                                   hipStream_t stream, int cooperative);
+__attribute__((visibility("hidden"))) int cell_launch(const Params& p, const void* region, hipStream_t stream,
+                                                   int cooperative);
 __attribute__((visibility("hidden"))) size_t cell_region_bytes();
 
 // ------------------------------------------------------------------------------------------------

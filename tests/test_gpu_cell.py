@@ -1,4 +1,4 @@
-"""The batched step of three or more sequences on cells of XCDs (decode_cell.hip): context lengths at the
+"""The batched step of three or more sequences (135M: on cells of XCDs, decode_cell.hip): context lengths at the
 edges of its tiles, quads, chunks and shares, every number of sequences a cell can hold, and caches laid
 out otherwise.  Bars as in test_gpu_batched.py (or twice the eager-GPU floor of the
 same sequence)."""
