@@ -82,7 +82,8 @@ PyObject* step(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* fn = address(0);
   void* stream = address(1);
   const auto* s = static_cast<const Spec*>(PyCapsule_GetPointer(a[2], kSpec));
-  const long nl = PyLong_AsLong(a[3]);
+  int overflow = 0;  // a count past a long is no error here: below it is out of range
+  const long nl = PyLong_AsLongAndOverflow(a[3], &overflow);
   const int want_ids = PyObject_IsTrue(a[16]);
   void *out = address(17), *ids = address(18), *scratch = address(19);
   const size_t scratch_bytes = PyLong_AsSize_t(a[20]);
