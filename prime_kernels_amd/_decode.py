@@ -95,7 +95,8 @@ class _Runtime:
         self.layers_t = None
         self.kv_t = None
         self.table_key = None   # the addresses in the tables, layers then caches, as bytes
-        self.spec = _native.host().make_spec(
+        host = _native.host()
+        self.spec = None if host is None else host.make_spec(
             model.model_id, model.hidden, model.kv_heads, model.head_dim, model.max_batch, model.max_seq, model.layers,
             VOCAB, BLOCK_SIZE, [(dtype == torch.bfloat16, shape) for _, dtype, shape in model.layer_spec()])
         self.entry = _native.entry_address("pk_decode_mxfp8" if model.weight_format == "mxfp8" else "pk_decode")
@@ -242,7 +243,7 @@ def decode_step(model: Model, *, input_ids, positions, seq_lens, block_table, sl
     weights of every enabled layer."""
     nl = model.layers if num_layers is None else int(num_layers)
     rt = _runtimes.get((model.name, input_ids.device)) if type(input_ids) is torch.Tensor else None
-    if rt is not None and debug is None and eps == EPS and -1 <= debug_layer_index < model.layers and (
+    if rt is not None and rt.spec is not None and debug is None and eps == EPS and -1 <= debug_layer_index < model.layers and (
             encoded_gu is None or (model.model_id == 360 and model.weight_format == "bf16" and encoded_gu.device == rt.device)):
         rc = _plain_step(rt, model, nl, encoded_gu, return_token_ids or logits_out is not None, input_ids, positions,
                          seq_lens, block_table, slot_mapping, embed, layers, final_norm, kv_caches, cos_sin_cache,

@@ -1,8 +1,9 @@
 """ctypes binding of the C ABI in include/prime_decode.h (libprime_decode.so), and the host module
 that checks and launches a decode step (csrc/host_step.cpp).
 
-This is the only place Python crosses into native code.  There is no fallback: if either is
-missing its first use raises.
+This is the only place Python crosses into native code.  There is no fallback for the library: if it
+is missing its first use raises.  The host module is compiled against one torch and one Python; under
+others decode_step makes the same checks in Python.
 """
 
 from __future__ import annotations
@@ -10,10 +11,11 @@ from __future__ import annotations
 import ctypes
 import importlib.machinery
 import importlib.util
+import sysconfig
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libprime_decode.so"
-HOST_PATH = LIB_PATH.with_name("_host_step.so")
 
 MODEL_360M = 360
 MODEL_135M = 135
@@ -107,19 +109,31 @@ def status_string(rc: int) -> str:
     return library().prime_decode_status_string(rc).decode()
 
 
+def host_path(torch_version: str) -> Path:
+    """The host module built against `torch_version` and this Python: its C++ interfaces are those of that
+    torch alone, so the file's name says which."""
+    return LIB_PATH.with_name(f"_host_step-torch{torch_version}.{sysconfig.get_config_var('SOABI')}.so")
+
+
 def host():
-    """The host module: make_spec and step (csrc/host_step.cpp)."""
+    """The host module, make_spec and step (csrc/host_step.cpp), or None (with one warning) when there is
+    no build of it for the running torch and Python: decode_step then checks in Python, for about 200 us
+    more a call."""
     global _host
     if _host is None:
-        if not HOST_PATH.is_file():
-            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -m prime_kernels_amd.build`")
-        import torch  # noqa: F401  (the module links against torch's libraries)
+        import torch
 
-        loader = importlib.machinery.ExtensionFileLoader("_host_step", str(HOST_PATH))
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_host_step", loader))
-        loader.exec_module(module)
-        _host = module
-    return _host
+        path = host_path(torch.__version__)
+        if path.is_file():
+            loader = importlib.machinery.ExtensionFileLoader("_host_step", str(path))
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_host_step", loader))
+            loader.exec_module(module)
+            _host = module
+        else:
+            warnings.warn(f"{path} is missing: decode_step checks its arguments in Python; build it with "
+                          "`python -m prime_kernels_amd.build`", RuntimeWarning, stacklevel=2)
+            _host = False
+    return _host or None
 
 
 def entry_address(name: str) -> int:

@@ -1,5 +1,5 @@
 """Build the native library `_lib/libprime_decode.so` with hipcc for gfx950, and the host module
-`_lib/_host_step.so`.
+`_lib/_host_step-*.so` for the installed torch.
 
 Usage: python -m prime_kernels_amd.build   (also called by __graft_entry__.build()).
 The library is built in-tree so it travels with the source tree; nothing is JIT-compiled at
@@ -22,7 +22,6 @@ LIB = LIB_DIR / "libprime_decode.so"
 SOURCES = [PKG / "csrc" / "decode_megakernel.hip", PKG / "csrc" / "decode_sr.hip", PKG / "csrc" / "decode_cell.hip",
            PKG / "csrc" / "lossless_bf16.hip"]
 HOST_SOURCE = PKG / "csrc" / "host_step.cpp"
-HOST_LIB = LIB_DIR / "_host_step.so"
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [
@@ -40,6 +39,15 @@ def hipcc() -> str:
         if cand and Path(cand).exists():
             return cand
     raise RuntimeError("hipcc not found")
+
+
+def host_compiler() -> str:
+    """A C++ compiler for host code: $CXX, the system's, or the clang that hipcc drives."""
+    for cand in (os.environ.get("CXX"), "g++", "c++", str(Path(hipcc()).with_name("amdclang++")), "/opt/rocm/bin/amdclang++"):
+        found = shutil.which(cand) if cand else None
+        if found:
+            return found
+    raise RuntimeError("no C++ compiler found for the host module")
 
 
 def build(verbose: bool = False) -> Path:
@@ -60,10 +68,13 @@ def build_host(verbose: bool = False) -> Path:
     """The Python module of the step's argument checks (host code only), against the installed torch."""
     import torch
 
+    from prime_kernels_amd import _native
+
+    host_lib = _native.host_path(torch.__version__)
     torch_dir = Path(torch.__file__).resolve().parent
     lib = torch_dir / "lib"
-    tmp = HOST_LIB.with_suffix(".so.tmp")
-    cmd = [os.environ.get("CXX") or shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
+    tmp = host_lib.with_suffix(".so.tmp")
+    cmd = [host_compiler(), "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{torch_dir / 'include'}",
            f"-I{torch_dir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}", f"-I{sysconfig.get_paths()['include']}",
            str(HOST_SOURCE), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", f"-Wl,-rpath,{lib}", "-o", str(tmp)]
@@ -72,8 +83,8 @@ def build_host(verbose: bool = False) -> Path:
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"{cmd[0]} failed ({res.returncode}):\n{res.stderr[-4000:]}")
-    os.replace(tmp, HOST_LIB)
-    return HOST_LIB
+    os.replace(tmp, host_lib)
+    return host_lib
 
 
 if __name__ == "__main__":

@@ -1,6 +1,7 @@
 """The host module of the step's checks (csrc/host_step.cpp) without a GPU: it answers None for whatever it
 does not find right, so that decode_step's own checks word the error."""
 
+import pytest
 import torch
 
 from prime_kernels_amd import _decode, _native
@@ -20,3 +21,14 @@ def _call(n_layers):
 def test_layer_counts_of_any_size_are_left_to_the_python_checks():
     for n in (0, -1, 32, 2 ** 31, 2 ** 63, 2 ** 70, -2 ** 70):
         assert _call(n) is None, n
+
+
+def test_another_torch_gets_no_host_module(monkeypatch):
+    """The module is built against one torch's C++ interfaces: under another version there is none, with a
+    warning and no error, and the build for this version is found by its own name."""
+    assert _native.host_path(torch.__version__).is_file() and _native.host() is not None
+    monkeypatch.setattr(_native, "_host", None)
+    monkeypatch.setattr(torch, "__version__", "0.0.1")
+    with pytest.warns(RuntimeWarning, match="checks its arguments in Python"):
+        assert _native.host() is None
+    assert _native.host() is None

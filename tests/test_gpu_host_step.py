@@ -68,6 +68,23 @@ def test_both_paths_give_the_same_bits(batch):
     assert torch.equal(h, one[0]) and torch.equal(ids, one[1].float().argmax(-1))
 
 
+def test_without_the_host_module_the_same_bits(monkeypatch):
+    """A torch that the host module was not built for: decode_step checks and launches from Python."""
+    _need_gpu()
+    from prime_kernels_amd import _decode, _native
+
+    mod, kw = _arguments(3)
+    mod.decode_step(**kw)
+    one = _clone(kw, mod.decode_step(**kw))
+    monkeypatch.setattr(_native, "_host", False)
+    monkeypatch.setattr(_decode, "_runtimes", {})
+    mod.decode_step(**kw)
+    two = _clone(kw, mod.decode_step(**kw))
+    assert all(torch.equal(a, b) for a, b in zip(one, two))
+    with pytest.raises(ValueError, match="positions must have dtype"):
+        mod.decode_step(**dict(kw, positions=kw["positions"].int()))
+
+
 def test_every_wrong_argument_is_refused():
     _need_gpu()
     mod, kw = _arguments()
