@@ -12,6 +12,7 @@ and the tied LM head stay bf16.
 from __future__ import annotations
 
 import ctypes
+import itertools
 
 import torch
 
@@ -58,10 +59,14 @@ def quantize(w: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
 def quantize_layers(layers) -> list[tuple]:
     """bf16 layer tuples (norm1, qkv, o, norm2, gate_up, down) -> MXFP8 layer tuples
     (norm1, qkv, qkv_scales, o, o_scales, norm2, gate_up, gate_up_scales, down, down_scales)."""
-    layers = [tuple(layer) for layer in layers]
-    done = iter(_quantize_all([w for _, qkv, o, _, gate_up, down in layers for w in (qkv, o, gate_up, down)]))
+    # A list's layers are there anyway: eight of them, 32 matrices, are one launch.  What an iterator makes
+    # is taken layer by layer, so that each can be freed before the next is made.
+    group = 8 if isinstance(layers, (list, tuple)) else 1
+    source = iter(layers)
     out = []
-    for norm1, _, _, norm2, _, _ in layers:
-        (q1, s1), (q2, s2), (q3, s3), (q4, s4) = next(done), next(done), next(done), next(done)
-        out.append((norm1, q1, s1, q2, s2, norm2, q3, s3, q4, s4))
+    while taken := [tuple(layer) for layer in itertools.islice(source, group)]:
+        done = iter(_quantize_all([w for _, qkv, o, _, gate_up, down in taken for w in (qkv, o, gate_up, down)]))
+        for norm1, _, _, norm2, _, _ in taken:
+            (q1, s1), (q2, s2), (q3, s3), (q4, s4) = next(done), next(done), next(done), next(done)
+            out.append((norm1, q1, s1, q2, s2, norm2, q3, s3, q4, s4))
     return out
