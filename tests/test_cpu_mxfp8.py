@@ -36,8 +36,8 @@ def test_layers_of_an_iterator_are_taken_one_at_a_time(monkeypatch):
     assert taken == [4] * 12 and most <= 1
 
 
-def test_layers_of_a_list_go_eight_at_a_time(monkeypatch):
-    """32 matrices a launch, so that the copies of strided ones are no more than one launch's."""
+def test_layers_of_a_list_go_32_at_a_time(monkeypatch):
+    """One call a model, and a bound on the copies that strided matrices need."""
     taken = []
 
     def matrices(ms):
@@ -46,11 +46,11 @@ def test_layers_of_a_list_go_eight_at_a_time(monkeypatch):
         return [(w, w) for w in ms]
 
     monkeypatch.setattr(mxfp8, "_quantize_all", matrices)
-    layers = [tuple(torch.full((1,), 10.0 * i + k) for k in range(6)) for i in range(19)]
+    layers = [tuple(torch.full((1,), 10.0 * i + k) for k in range(6)) for i in range(67)]
     for given in (layers, tuple(layers), [list(x) for x in layers]):
         taken.clear()
         out = mxfp8.quantize_layers(given)
-        assert taken == [32, 32, 12] and len(out) == 19
+        assert taken == [128, 128, 12] and len(out) == 67
         for x, (n1, q, _, o, _, n2, g, _, d, _) in zip(layers, out):
             assert all(a is b for a, b in zip((n1, q, o, n2, g, d), x))
     assert mxfp8.quantize_layers([]) == []
