@@ -12,6 +12,7 @@ and the tied LM head stay bf16.
 from __future__ import annotations
 
 import ctypes
+import functools
 import itertools
 
 import torch
@@ -22,52 +23,53 @@ from prime_kernels_amd._decode import mxfp8_scale_stride as scale_stride
 __all__ = ["quantize", "quantize_layers", "scale_stride"]
 
 
-def _size(w) -> tuple[int, int]:
-    if not isinstance(w, torch.Tensor) or not w.is_cuda or w.dtype != torch.bfloat16 or w.ndim != 2:
-        raise ValueError("w must be a 2-D bf16 CUDA tensor")
-    rows, cols = w.shape
-    if cols % 32 or cols < 32:
-        raise ValueError("cols must be a positive multiple of 32")
-    return rows, cols
-
-
-def _raise_on(rc: int) -> None:
-    if rc != 0:
-        raise RuntimeError(f"MXFP8 quantisation failed: {_native.status_string(rc)}")
-
-
 def _quantize_all(matrices) -> list[tuple[torch.Tensor, torch.Tensor]]:
     """(codes, scales) of each matrix, all of one device in one call of the library."""
     checked, devices = [], {}
     for w in matrices:
-        rows, cols = _size(w)
+        if not isinstance(w, torch.Tensor) or not w.is_cuda or w.dtype != torch.bfloat16 or w.ndim != 2:
+            raise ValueError("w must be a 2-D bf16 CUDA tensor")
+        rows, cols = w.shape
+        if cols % 32 or cols < 32:
+            raise ValueError("cols must be a positive multiple of 32")
         devices.setdefault(w.device, []).append(len(checked))
-        checked.append((w.contiguous(), rows, cols))
+        # new_empty is the quicker one, but a subclass's gives the subclass
+        new = w.new_empty if type(w) is torch.Tensor else functools.partial(torch.empty, device=w.device)
+        checked.append((w.contiguous(), new, rows, cols))
     lib = _native.library()
-    out = [(w.new_empty((rows, cols), dtype=torch.uint8), w.new_empty((rows, scale_stride(cols)), dtype=torch.uint8))
-           for w, rows, cols in checked]
+    out = [(new((rows, cols), dtype=torch.uint8), new((rows, scale_stride(cols)), dtype=torch.uint8))
+           for _, new, rows, cols in checked]
     for device, mine in devices.items():
         n = len(mine)
         pointers, ints = ctypes.c_void_p * n, ctypes.c_int * n
         with torch.cuda.device(device):
-            _raise_on(lib.pk_quantize_mxfp8_many(
+            rc = lib.pk_quantize_mxfp8_many(
                 torch.cuda.current_stream(device).cuda_stream, n,
                 pointers(*[checked[i][0].data_ptr() for i in mine]), pointers(*[out[i][0].data_ptr() for i in mine]),
-                pointers(*[out[i][1].data_ptr() for i in mine]), ints(*[checked[i][1] for i in mine]),
-                ints(*[checked[i][2] for i in mine])))
+                pointers(*[out[i][1].data_ptr() for i in mine]), ints(*[checked[i][2] for i in mine]),
+                ints(*[checked[i][3] for i in mine]))
+        if rc != 0:
+            raise RuntimeError(f"MXFP8 quantisation failed: {_native.status_string(rc)}")
     return out
 
 
 def quantize(w: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """bf16 CUDA matrix [rows, cols] -> (e4m3 codes, e8m0 scales) on the same device, computed by
     the library's quantisation kernel on the current stream."""
-    rows, cols = _size(w)
+    if not isinstance(w, torch.Tensor) or not w.is_cuda or w.dtype != torch.bfloat16 or w.ndim != 2:
+        raise ValueError("w must be a 2-D bf16 CUDA tensor")
+    rows, cols = w.shape
+    if cols % 32 or cols < 32:
+        raise ValueError("cols must be a positive multiple of 32")
     w = w.contiguous()
     q = torch.empty((rows, cols), dtype=torch.uint8, device=w.device)
     s = torch.empty((rows, scale_stride(cols)), dtype=torch.uint8, device=w.device)
+    lib = _native.library()
     with torch.cuda.device(w.device):
-        _raise_on(_native.library().pk_quantize_mxfp8(torch.cuda.current_stream(w.device).cuda_stream, w.data_ptr(), q.data_ptr(),
-                                                      s.data_ptr(), rows, cols))
+        rc = lib.pk_quantize_mxfp8(torch.cuda.current_stream(w.device).cuda_stream, w.data_ptr(), q.data_ptr(),
+                                   s.data_ptr(), rows, cols)
+    if rc != 0:
+        raise RuntimeError(f"MXFP8 quantisation failed: {_native.status_string(rc)}")
     return q, s
 
 

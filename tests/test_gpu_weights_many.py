@@ -56,6 +56,24 @@ def test_quantizer_many_matrices():
         assert np.array_equal(q.cpu().numpy(), q_ref) and np.array_equal(s.cpu().numpy(), s_ref), tuple(w.shape)
 
 
+class _Other(torch.Tensor):
+    """A subclass, as a program's own parameter type may be."""
+
+
+def test_quantizer_gives_plain_tensors():
+    """The codes and scales of a subclass's matrix are plain tensors, one matrix or many, strided or not."""
+    _need_gpu()
+    from prime_kernels_amd import mxfp8
+
+    w = (torch.randn((64, 96), generator=torch.Generator().manual_seed(1)) * 0.02).to(torch.bfloat16).cuda()
+    wide = torch.stack((w, -w), dim=2).view(64, 192)[:, ::2]
+    want = mxfp8.quantize(w)
+    for given in (w, wide, w.as_subclass(_Other), wide.as_subclass(_Other), torch.nn.Parameter(w, requires_grad=False)):
+        layer = (None, given, given, None, given, given)
+        for got in (mxfp8.quantize(given), mxfp8._quantize_all([given])[0], mxfp8.quantize_layers([layer])[0][6:8]):
+            assert all(type(g) is torch.Tensor and torch.equal(g, t) for g, t in zip(got, want))
+
+
 @pytest.mark.parametrize("layers", [1, 33])
 def test_lossless_encode_layers_equals_one_by_one(layers):
     """Layers with few, no and only escapes, tables too small for theirs, in one call (32 layers a launch):
