@@ -92,13 +92,14 @@ class _Runtime:
         self.scratch_bytes = nbytes
         self.out = torch.empty((model.max_batch, model.hidden), dtype=torch.bfloat16, device=device)
         self.ids = torch.empty((model.max_batch,), dtype=torch.int64, device=device)
+        self.layer_spec = model.layer_spec()
         self.layers_t = None
         self.kv_t = None
         self.table_key = None   # the addresses in the tables, layers then caches, as bytes
         host = _native.host()
         self.spec = None if host is None else host.make_spec(
             model.model_id, model.hidden, model.kv_heads, model.head_dim, model.max_batch, model.max_seq, model.layers,
-            VOCAB, BLOCK_SIZE, [(dtype == torch.bfloat16, shape) for _, dtype, shape in model.layer_spec()])
+            VOCAB, BLOCK_SIZE, [(dtype == torch.bfloat16, shape) for _, dtype, shape in self.layer_spec])
         self.entry = _native.entry_address("pk_decode_mxfp8" if model.weight_format == "mxfp8" else "pk_decode")
         self.entry_encoded = _native.entry_address("pk_decode_lossless")
 
@@ -189,11 +190,11 @@ def _tables(rt: _Runtime, layers, kv_caches):
     return rt.layers_t, rt.kv_t
 
 
-def _plain_step(rt: _Runtime, model: Model, nl: int, encoded_gu, want_ids, input_ids, positions, seq_lens, block_table,
+def _plain_step(rt: _Runtime, stream: int, nl: int, encoded_gu, want_ids, input_ids, positions, seq_lens, block_table,
                 slot_mapping, embed, layers, final_norm, kv_caches, cos_sin_cache, layer_outputs, logits_out):
     """Check and launch in the host module: the entry point's status, or None when an argument is not
     plainly right (decode_step's own checks then decide)."""
-    step, stream = _native.host().step, torch.cuda.current_stream(rt.device).cuda_stream
+    step = _native.host().step
     for _ in range(2):
         r = step(rt.entry if encoded_gu is None else rt.entry_encoded, stream, rt.spec, nl, input_ids, positions, seq_lens,
                  slot_mapping, block_table, embed, final_norm, layers, kv_caches, cos_sin_cache, layer_outputs, logits_out,
@@ -243,9 +244,11 @@ def decode_step(model: Model, *, input_ids, positions, seq_lens, block_table, sl
     weights of every enabled layer."""
     nl = model.layers if num_layers is None else int(num_layers)
     rt = _runtimes.get((model.name, input_ids.device)) if type(input_ids) is torch.Tensor else None
+    stream = None
     if rt is not None and rt.spec is not None and debug is None and eps == EPS and -1 <= debug_layer_index < model.layers and (
             encoded_gu is None or (model.model_id == 360 and model.weight_format == "bf16" and encoded_gu.device == rt.device)):
-        rc = _plain_step(rt, model, nl, encoded_gu, return_token_ids or logits_out is not None, input_ids, positions,
+        stream = torch.cuda.current_stream(rt.device).cuda_stream
+        rc = _plain_step(rt, stream, nl, encoded_gu, return_token_ids or logits_out is not None, input_ids, positions,
                          seq_lens, block_table, slot_mapping, embed, layers, final_norm, kv_caches, cos_sin_cache,
                          layer_outputs, logits_out)
         if rc is not None:
@@ -288,11 +291,14 @@ def decode_step(model: Model, *, input_ids, positions, seq_lens, block_table, sl
     _check_tensor(final_norm, "final_norm", dtype=torch.bfloat16, device=device, shape=(model.hidden,))
     check_embed_shape(embed, model)
     lm_head = return_token_ids or logits_out is not None
-    spec = model.layer_spec()
+    spec = rt.layer_spec if rt is not None else model.layer_spec()
     for i, layer in enumerate(layers):
         if len(layer) != len(spec):
             raise ValueError(f"layer {i} must contain {'six' if len(spec) == 6 else len(spec)} weight tensors")
         for (name, dtype, shape), tensor in zip(spec, layer):
+            if isinstance(tensor, torch.Tensor) and tensor.is_cuda and tensor.dtype == dtype and tensor.device == device \
+                    and tuple(tensor.shape) == shape and tensor.is_contiguous() and tensor.data_ptr() % 16 == 0:
+                continue
             _check_tensor(tensor, f"layer {i} {name}", dtype=dtype, device=device, shape=shape)
             if not tensor.is_contiguous():
                 raise ValueError(f"layer {i} {name} must be contiguous")
@@ -342,7 +348,8 @@ def decode_step(model: Model, *, input_ids, positions, seq_lens, block_table, sl
 
     rt = runtime(model, device)
     layers_t, kv_t = _tables(rt, layers, kv_caches)
-    stream = torch.cuda.current_stream(device).cuda_stream
+    if stream is None:
+        stream = torch.cuda.current_stream(device).cuda_stream
     want_ids = return_token_ids or logits_out is not None
     if debug is not None:
         launch = rt.lib.pk_decode_debug
