@@ -54,6 +54,8 @@ int lossless_encode_layer(const void* input, void* plane, void* headers, void* r
 
 /* Encode `layers` matrices, 32 a launch (host arrays of one entry per layer, the buffers as above);
  * totals [layers] receives each layer's escaped chunks.  Nothing is launched when a layer is refused.
+ * The workspace belongs to the call until it has run: a layer whose encoding another call in the same
+ * workspace upset may end disabled with a total of ~0.
  * No reference counterpart. */
 size_t lossless_encode_workspace_bytes(int layers);
 int lossless_encode_layers(int layers, const void* const* input, void* const* plane, void* const* headers,

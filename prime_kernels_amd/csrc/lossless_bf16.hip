@@ -170,11 +170,12 @@ struct LayerArgs {
 };
 struct BatchArgs {
   LayerArgs l[kBatch];
-  uint64_t* states;       // [layers][kBlocks]: kAggregate or kPrefix in the upper half, the count in the lower
+  uint64_t* states;       // [layers][kBlocks]: kAggregate, kPrefix or kFailed in the upper half, the count in the lower
   uint32_t* tickets;      // [layers]
   uint32_t* totals;       // [layers]
 };
-constexpr uint64_t kAggregate = 1ull << 32, kPrefix = 2ull << 32;
+constexpr uint64_t kAggregate = 1ull << 32, kPrefix = 2ull << 32, kFailed = 3ull << 32;
+constexpr int kScanPolls = 1 << 22;  // seconds; a wait takes microseconds
 
 __global__ void __launch_bounds__(256) lz_clear(uint64_t* states, uint32_t* tickets, int layers) {
   const int i = blockIdx.x * 256 + threadIdx.x;
@@ -185,6 +186,9 @@ __global__ void __launch_bounds__(256) lz_clear(uint64_t* states, uint32_t* tick
 // One pass with a decoupled look-back scan.  A workgroup takes its rows by ticket, so the workgroups whose
 // counts it waits for have started before it and wait only for earlier ones: every wait ends.  It publishes its
 // count, adds up its predecessors' (64 states at a time) until it meets a prefix, and publishes its own.
+// That holds while the pass has its workspace to itself.  Another pass in it would hand out tickets past the last
+// rows and clear states that are waited for: a workgroup without rows does nothing, and a wait that is too long
+// gives up, which its successors take over, so that the layer ends disabled with a total of ~0.
 // 32 layers of random weights (315 MB read, 236 MB written) take 168 us (3.3 TB/s), a call 219; counting
 // first and placing the escapes in a later kernel took 98 + 5 + 67 (scattered 4-byte header writes, a second
 // read of the escaped chunks), a call 257, and three launches and a copy for each layer 621.
@@ -195,6 +199,7 @@ __global__ void __launch_bounds__(64 * kWavesPerBlock) lz_encode_many(BatchArgs 
   if (threadIdx.x == 0) ticket = __hip_atomic_fetch_add(a.tickets + blockIdx.y, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   const int block = __builtin_amdgcn_readfirstlane(int(ticket));
+  if (block >= kBlocks) return;
   const int row0 = block * kRowsPerBlock + wave * kRowsPerWave;
   const bool second = lane + 64 < kChunksPerRow;
   uint4 v[kRowsPerWave][2];
@@ -226,31 +231,36 @@ __global__ void __launch_bounds__(64 * kWavesPerBlock) lz_encode_many(BatchArgs 
 #pragma unroll
     for (int w = 0; w < kWavesPerBlock; ++w) mine += wave_count[w];
     uint32_t before = 0;
+    bool failed = false;
     if (block > 0) {
       if (lane == 0) __hip_atomic_store(states + block, kAggregate | mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       for (int top = block;;) {  // states top - 1 (lane 0) .. top - 64
         const int at = top - 1 - lane;
         uint64_t st = kPrefix;  // before the first workgroup: a prefix of zero
-        if (at >= 0)
+        if (at >= 0) {
+          int polls = 0;
           do st = __hip_atomic_load(states + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          while (st == 0ull);
-        const uint64_t prefix = __ballot((st >> 32) == 2ull);
+          while (st == 0ull && ++polls < kScanPolls);
+          if (st == 0ull) st = kFailed;
+        }
+        const uint64_t prefix = __ballot((st >> 32) >= 2ull);
         const int last = prefix ? __builtin_ctzll(prefix) : 63;  // nearest prefix; the aggregates before it add up
         uint32_t x = lane <= last ? uint32_t(st) : 0u;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
         before += x;
+        failed = __ballot(lane == last && st >= kFailed) != 0ull;
         if (prefix) break;
         top -= 64;
       }
     }
     if (lane == 0) {
-      __hip_atomic_store(states + block, kPrefix | (before + mine), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(states + block, failed ? kFailed : kPrefix | (before + mine), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       before_block = before;
       if (block == kBlocks - 1) {
-        const uint32_t total = before + mine;
+        const uint32_t total = failed ? ~0u : before + mine;
         L.row_offsets[kRows] = total;
-        *L.enabled = total <= L.capacity ? 1u : 0u;
+        *L.enabled = total <= L.capacity && !failed ? 1u : 0u;
         a.totals[blockIdx.y] = total;
       }
     }

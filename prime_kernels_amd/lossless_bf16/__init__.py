@@ -19,6 +19,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import threading
 from dataclasses import dataclass
 
 import torch
@@ -68,6 +69,7 @@ class EncodedGUCache:
         # the encoder's scratch: its scan states
         self._scan_bytes = self._lib.lossless_encode_workspace_bytes(LAYERS)
         self._scan = torch.empty((self._scan_bytes,), dtype=torch.uint8, device=dev)
+        self._lock = threading.Lock()  # one pass at a time: its workgroups wait for each other through the scratch
         self._counts = torch.empty((LAYERS,), dtype=u32, device=dev)
         self._layers = [
             _LayerCode(plane=torch.empty((ROWS, COLS), dtype=torch.uint8, device=dev),
@@ -130,8 +132,11 @@ class EncodedGUCache:
             rc = self._lib.lossless_encode_layers(LAYERS, column(weights), *self._columns, (ctypes.c_uint32 * LAYERS)(*capacities),
                                                   self._counts.data_ptr(), self._scan.data_ptr(), self._scan_bytes,
                                                   stream.cuda_stream)
-        _raise_on(rc, "encode")
-        return self._counts.view(torch.int32).tolist()  # waits for the pass
+        _raise_on(rc, f"encode layers 0..{LAYERS - 1}")
+        counts = self._counts.view(torch.int32).tolist()  # waits for the pass
+        if min(counts) < 0:
+            raise RuntimeError(f"lossless gate/up cache: encode layer {counts.index(min(counts))}: gave up a wait")
+        return counts
 
     @torch.inference_mode()
     def refresh(self, weights) -> None:
@@ -143,12 +148,13 @@ class EncodedGUCache:
         self._check(weights)
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("the lossless gate/up cache cannot be refreshed during graph capture")
-        torch.cuda.synchronize(self.device)
-        counts = self._encode_pass(weights, [c.capacity for c in self._layers])
-        for code, n in zip(self._layers, counts):
-            code.found = n
-        self._weights = weights
-        self.generation += 1
+        with self._lock:
+            torch.cuda.synchronize(self.device)
+            counts = self._encode_pass(weights, [c.capacity for c in self._layers])
+            for code, n in zip(self._layers, counts):
+                code.found = n
+            self._weights = weights
+            self.generation += 1
 
     # -- state ------------------------------------------------------------------------------------
 

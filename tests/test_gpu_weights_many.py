@@ -135,3 +135,39 @@ def test_lossless_encode_layers_equals_one_by_one(layers):
         assert int(got[i]) == totals[i % kinds], i
         for k, v in b.items():
             assert torch.equal(v, one[i % kinds][k]), (i, k)
+
+
+def test_refreshes_of_one_cache_from_two_threads():
+    """Each thread on its own stream with its own weights, the passes one after the other: the cache ends as
+    the encoding of the weights it says it holds, and no pass is lost."""
+    _need_gpu()
+    import threading
+
+    from prime_kernels_amd.lossless_bf16 import LAYERS, EncodedGUCache
+
+    def matrices(seed, std):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        return [(torch.randn((5120, 960), generator=g, device="cuda") * std).to(torch.bfloat16) for _ in range(LAYERS)]
+
+    sets = [matrices(1, 0.02), matrices(2, 0.021)]
+    cache = EncodedGUCache(sets[0])
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(weights):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(5):
+                    cache.refresh(weights)
+        except Exception as e:  # noqa: BLE001 - shown by the assertion below
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(w,)) for w in sets]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    assert cache.generation == 11 and cache.statistics()["active_layers"] == LAYERS
+    for i in range(LAYERS):
+        assert cache.enabled(i) and torch.equal(cache.decode_layer(i).view(torch.int16), cache.weights[i].view(torch.int16)), i
