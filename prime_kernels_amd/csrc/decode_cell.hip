@@ -26,10 +26,11 @@
 //
 // Exchange format: 16-byte units {two 32-bit words of payload (four bf16, the four consecutive rows
 // a lane holds after v_mfma_f32_16x16x32_bf16) or three fp32 words, 32-bit tag}, one store and one
-// load each (never seen torn: test_gpu_safety.py::test_exchange_units_are_never_torn).  A tag is
-// (step epoch << 5) | layer: the buffers are reused by every layer, which is safe because a buffer
-// can only be written for layer l + 1 after every workgroup of the cell has read it for layer l
-// (each exchange waits for units that depend on all of the previous exchange's readers).
+// load each (never seen torn: test_gpu_safety.py::test_exchange_units_are_never_torn).  The buffers
+// are reused by every layer, which is safe because a buffer can only be written for layer l + 1 after
+// every workgroup of the cell has read it for layer l (each exchange waits for units that depend on all
+// of the previous exchange's readers).  A unit of two payload words says its layer and step epoch; one
+// of three has a single word for both (CC::tag).
 //
 // Rounding points are those of HF eager Llama (modeling_llama.py), as in the other kernels.
 #include <hip/hip_runtime.h>
@@ -101,9 +102,9 @@ struct CG {
 
 // Exchange region (units of 16 bytes from its base; one layout for both splits of the pairs, so that no unit is
 // read in a format it was not written in): the workgroups' end records per sequence (tag: epoch), the
-// vectors per sequence (tag: epoch, and the layer in the word before it; the attention vector: (epoch << 5) |
-// layer), the attention records of each workgroup's items (statistics, 2 units; partial sums, 64 units; the
-// same tag).
+// vectors per sequence (tag: epoch, and the layer in the word before it; the attention vector: CC::tag), the
+// attention records of each workgroup's items (statistics, 2 units; partial sums, 64 units; CC::tag).
+// The vectors and records are there twice, the second copy for some attentions' units (CC::copy).
 enum CKind { C_X, C_ATT, C_H1, C_QKV, C_ACT };
 template <class G>
 struct CW {
@@ -114,8 +115,8 @@ struct CW {
   static constexpr uint32_t UPL = PK_CELL_UPL, LINES = (640 + UPL - 1) / UPL, SLOTS = BMAX * 5 + 1;
   static_assert(HU <= 640 && QU <= 640 && IU <= 640, "a vector's lines");
   static constexpr uint32_t REC0 = V0 + LINES * SLOTS * 4;
-  static constexpr uint32_t REC = 66;
-  static constexpr uint32_t TOTAL = REC0 + uint32_t(NWG) * IPW_MAX * REC;
+  static constexpr uint32_t REC = 66, END = REC0 + uint32_t(NWG) * IPW_MAX * REC;
+  static constexpr uint32_t COPY = END - V0, TOTAL = END + COPY;
   __device__ static uint32_t end(int b, int wg) { return (uint32_t(b) * NWG + uint32_t(wg)) * 16u; }
   // unit u of vector `kind` of sequence slot cs (cell * NS + slot): lane part and uniform part
   __device__ static uint32_t vec_u(int u) { return (V0 + uint32_t(u) / UPL * SLOTS * 4u + uint32_t(u) % UPL) * 16u; }
@@ -510,7 +511,18 @@ struct CC {
     ns = __builtin_amdgcn_readfirstlane(sm.ns);
   }
   __device__ __forceinline__ void refresh() { asm volatile("" : "+v"(lane), "+v"(ct)); }
-  __device__ __forceinline__ uint32_t tag(int l) const { return (epoch << 5) | uint32_t(l); }
+  // The attention's units hold three payload words and one for the epoch and the layer.  Every unit that a step uses
+  // is written and read by the same waves in each of its layers, so from a step's second layer on only the layer
+  // before it has to be told apart: odd layers flip the epoch's top bit.  At its first use in a step a unit may be
+  // as old as the program, so a step leaves none with the bit flipped: a last layer that is odd takes the second copy.
+  // The first use of either copy then finds whole epochs of other steps, as with the units that hold both words.
+  // (A step that gave up may leave a flipped one.)
+  uint32_t tag = 0, copy = 0;
+  __device__ __forceinline__ void begin_layer(int l) {
+    const bool odd = l & 1, last = l == p.n_layers - 1;
+    tag = epoch ^ (odd && !last ? 0x80000000u : 0u);
+    copy = odd && last ? W::COPY * 16u : 0u;
+  }
   __device__ __forceinline__ uint32_t filled() const {
     typedef __attribute__((address_space(3))) const volatile u32x4 lds_u32x4;
     const u32x4 f = *(lds_u32x4*)(sm.front);
@@ -725,19 +737,9 @@ __device__ __forceinline__ void stage_att_n(CC<G, PX>& C, int l) {
   using S = CG<G, PX>;
   u32x4 x[N];
   constexpr int AU = G::H / 6;
-  const uint32_t o = CW<G>::vec_u(min(C.ct, AU - 1)), tg = C.tag(l);
-  if constexpr (!S::E2E && S::NS > 4) {
-    // Workgroups with short chunks wait here while others still stream: for one unit, a sum of the longest
-    // chunk (the vectors follow it by an exchange), instead of up to 20 KB a try
-    const int slow = __builtin_amdgcn_readfirstlane(C.sm.slow);
-    if (slow >= 0) {
-      u32x4 y[1];
-      const uint32_t os = CW<G>::rec(C.P.cell * S::R + slow, 0, 2);
-      C.template poll<1>(55, 1u, [&](const u32x4& u) { return u.w == tg; }, [&](int) { return os; }, [&](int) { return 0u; }, y);
-    }
-  }
+  const uint32_t o = CW<G>::vec_u(min(C.ct, AU - 1)), tg = C.tag, copy = C.copy;
   C.template poll<N>(44 + C_ATT, (1u << C.ns) - 1u, [&](const u32x4& u) { return u.w == tg; }, [&](int) { return o; },
-                     [&](int i) { return CW<G>::vec_s(C_ATT, C.slot0() + i); }, x);
+                     [&](int i) { return CW<G>::vec_s(C_ATT, C.slot0() + i) + copy; }, x);
   if (C.ct < AU)
 #pragma unroll
     for (int i = 0; i < N; ++i)
@@ -943,7 +945,7 @@ __device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
   const int slot = C.slot0() + one(it.slot);
   const int nquad = (nt + 3) / 4;
   const int me = C.P.cell * S::R + C.P.r;
-  const uint32_t tg = C.tag(l);
+  const uint32_t tg = C.tag, copy = C.copy;
   const uint32_t kpos = C.pos, vpos = kpos + uint32_t(nt) * 2u * PKT;
   C.pos = vpos + uint32_t(nt) * 2u * PKT;
   const bool has_new = w == NCW - 1 && one(it.leader);  // the new token is wave 3's, in the chunk with the pair's end
@@ -1055,13 +1057,13 @@ __device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
       if (lane < 2)
         C.st(W::rec(me, 0, lane),
              lane == 0 ? u32x4{__float_as_uint(M[0]), __float_as_uint(M[1]), __float_as_uint(M[2]), tg}
-                       : u32x4{__float_as_uint(inv[0]), __float_as_uint(inv[1]), __float_as_uint(inv[2]), tg});
+                       : u32x4{__float_as_uint(inv[0]), __float_as_uint(inv[1]), __float_as_uint(inv[2]), tg}, copy);
     }
     tr(5);
     u32x4 y[2];
     const uint32_t o = W::rec(r0 + min(lane, Cc - 1), 0, 0);
     C.template poll<2>(51, 3u, [&](const u32x4& u) { return u.w == tg; }, [&](int i) { return o + 16u * uint32_t(i); },
-                       [&](int) { return 0u; }, y);
+                       [&](int) { return copy; }, y);
     const bool mine = lane < Cc;
     float mk[3];
 #pragma unroll
@@ -1162,7 +1164,7 @@ __device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
   C.release(C.pos);
   C.cbar();
   // ---- publish (wave 0): a pair in one chunk gives its attention values, others their fp32 partial sums ----
-  const uint32_t att = W::vec_s(C_ATT, slot);
+  const uint32_t att = W::vec_s(C_ATT, slot) + copy;
   if (w == 0) {
     skew_delay(p.skew, C.P.wg, l, 15);
     if (Cc > 1) {
@@ -1173,7 +1175,7 @@ __device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
 #pragma unroll
         for (int j = 0; j < NCW; ++j) v[i] += wo[j * 192 + 3 * lane + i];
       }
-      C.st(W::rec(me, 0, 2 + lane), u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), tg});
+      C.st(W::rec(me, 0, 2 + lane), u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), tg}, copy);
     } else if (lane < GRP) {
       float v[6];
 #pragma unroll
@@ -1197,7 +1199,7 @@ __device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
       u32x4 y[N];
       const int nc = min(N, Cc - c0);
       C.template poll<N>(52, (1u << nc) - 1u, [&](const u32x4& u) { return u.w == tg; }, [&](int) { return ou; },
-                         [&](int i) { return W::rec(r0 + c0 + i, 0, 0); }, y);
+                         [&](int i) { return W::rec(r0 + c0 + i, 0, 0) + copy; }, y);
 #pragma unroll
       for (int i = 0; i < N; ++i)
         if (i < nc) {
@@ -1225,7 +1227,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
   SmemC<G, PX>& sm = C.sm;
   const int lane = C.lane, w = C.cw;
   const int ni = __builtin_amdgcn_readfirstlane(sm.ni), ntile = __builtin_amdgcn_readfirstlane(sm.ntile);
-  const uint32_t tg = C.tag(l);
+  const uint32_t tg = C.tag, copy = C.copy;
   const int wgkey = C.P.cell * S::R;
   const uint32_t kpos = C.pos, vpos = kpos + uint32_t(ntile) * 2u * PKT;
   C.pos = vpos + uint32_t(ntile) * 2u * PKT;
@@ -1357,7 +1359,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
     if (sm.it[k].C > 1) {
       const u32x4 um = {__float_as_uint(rl(mx, 0)), __float_as_uint(rl(mx, 4)), __float_as_uint(rl(mx, 8)), tg};
       const u32x4 ul = {__float_as_uint(rl(ex, 0)), __float_as_uint(rl(ex, 4)), __float_as_uint(rl(ex, 8)), tg};
-      if (lane < 2) C.st(W::rec(wgkey + C.P.r, k, lane), lane == 0 ? um : ul);
+      if (lane < 2) C.st(W::rec(wgkey + C.P.r, k, lane), lane == 0 ? um : ul, copy);
     } else if (lane < 12 && (lane & 3) == 0) {
       sm.at.gml[k][lane >> 2] = mx;
       sm.at.gml[k][3 + (lane >> 2)] = 1.0f / ex;
@@ -1374,7 +1376,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) off[i] = int(W::rec(wgkey + r0 + c, c == 0 ? k0 : 0, i));
       C.template poll<2>(51, 3u, [&](const u32x4& u) { return u.w == tg; }, [&](int i) { return uint32_t(off[i]); },
-                         [&](int) { return 0u; }, x);
+                         [&](int) { return copy; }, x);
       const bool mine = lane < Cc;
       float M[3], mk[3], lk[3];
 #pragma unroll
@@ -1503,7 +1505,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
 #pragma unroll
         for (int x = 0; x < NCW; ++x) v[i] += o[x * 192 + 3 * lane + i];
       }
-      C.st(W::rec(wgkey + C.P.r, k, 2 + lane), u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), tg});
+      C.st(W::rec(wgkey + C.P.r, k, 2 + lane), u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), tg}, copy);
     } else if (lane < 32) {
       float v[6];
 #pragma unroll
@@ -1513,7 +1515,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
         for (int x = 0; x < NCW; ++x) v[i] += o[x * 192 + 6 * lane + i];
       }
       C.st(W::vec_u(sm.it[k].g * 32 + lane) + W::vec_s(C_ATT, slot0 + sm.it[k].slot),
-           u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), tg});
+           u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), tg}, copy);
     }
   }
   tr(7);
@@ -1533,7 +1535,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
         u32x4 x[N];
         const int n = min(N, Cc - c0);
         C.template poll<N>(52, (1u << n) - 1u, [&](const u32x4& u) { return u.w == tg; }, [&](int) { return o; },
-                           [&](int i) { return W::rec(r0 + c0 + i, c0 + i == 0 ? k0 : 0, 0); }, x);
+                           [&](int i) { return W::rec(r0 + c0 + i, c0 + i == 0 ? k0 : 0, 0) + copy; }, x);
 #pragma unroll
         for (int i = 0; i < N; ++i)
           if (i < n) {
@@ -1547,7 +1549,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
       for (int i = 0; i < 3; ++i) y[i] = dpp<0xb1>(0.f, v[i]);  // the pair's other lane
       if ((lane & 1) == 0 && lane < 2 * ng)
         C.st(W::vec_u(sm.it[k].g * 32 + g0 + (lane >> 1)) + W::vec_s(C_ATT, slot0 + sm.it[k].slot),
-             u32x4{pack2(v[0], v[1]), pack2(v[2], y[0]), pack2(y[1], y[2]), tg});
+             u32x4{pack2(v[0], v[1]), pack2(v[2], y[0]), pack2(y[1], y[2]), tg}, copy);
     }
   }
   C.cbar();  // the attention buffers share storage with the staged rows
@@ -1597,6 +1599,7 @@ __device__ __forceinline__ void consumer(const Params& p, const PlanC<G, PX>& P,
   for (int l = 0; l < p.n_layers && C.ns > 0; ++l) {
     // ---------------- RMSNorm(x) + QKV + RoPE ----------------
     C.refresh();
+    C.begin_layer(l);
     tr(l, 0);
     const NormW<G, PX> nw1(C);
     const Weights<S::KSH, S::TQ, G, PX> wq(C, (4 * nuq + 7) / 8);

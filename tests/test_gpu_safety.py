@@ -10,7 +10,8 @@
 * Exchange words carry the full 32-bit step epoch: steps that alternate batch sizes (so some words
   are not rewritten every step) give the same bits across the epoch's 32-bit wrap and across jumps
   of 65,536 and 65,535 epochs, where a 16-bit tag (with or without a skipped zero) would accept a
-  stale word as current.
+  stale word as current; 135M's batched kernel also across jumps of 2^27 and 2^31 epochs, where a tag of
+  (epoch << 5) | layer would.  (decode_kernel_b's softmax statistics and partial sums carry such a tag.)
 """
 
 import pytest
@@ -26,15 +27,19 @@ def _need_gpu():
         pytest.skip("no GPU")
 
 
-def _setup(batch_max, contexts, layers=2, seed=5):
+MODELS = {"360m": "decode_megakernel_360m", "135m": "decode_megakernel"}
+
+
+def _setup(batch_max, contexts, layers=2, seed=5, model="360m", capacity=None):
+    """`capacity`: tokens the block table addresses (default: the longest context + 64)."""
     import prime_kernels_amd as pk
     from prime_kernels_amd import workload as WL
 
-    mod = pk.load("decode_megakernel_360m")
+    mod = pk.load(MODELS[model])
     model = mod.MODEL
     dev = torch.device("cuda:0")
     embed, final_norm, lw = WL.random_weights(model, seed, dev, layers=layers)
-    cap = max(contexts) + 64
+    cap = capacity or max(contexts) + 64
     kv = WL.PagedKV(model, batch_max, cap, layers=layers, device=dev, seed=seed + 1, fill="randn")
     cos_sin = WL.rope_table(cap + 64, device=dev)
     return mod, model, embed, final_norm, lw, kv, cos_sin
@@ -114,16 +119,28 @@ def test_abandoned_wait_poisons_outputs_and_is_reported(path, report):
 
 
 def test_epoch_wrap_and_16_bit_jumps_with_alternating_batches():
+    _epoch_jumps("360m", None, 2, [65536, 65535, 65536, 65535])
+
+
+@pytest.mark.parametrize("layers", [1, 2, 3])
+@pytest.mark.parametrize("capacity", [None, 3904], ids=["whole_workgroups", "end_to_end"])
+def test_epoch_wrap_and_long_jumps_of_the_cell_kernel(capacity, layers):
+    """Both splits of 135M's batched kernel (16 * 3,904 tokens of block table are past 61,440), with a last
+    layer of either parity (the attention's units say the layer by one bit)."""
+    _epoch_jumps("135m", capacity, layers, [2 ** 27, 65535, 2 ** 31, 2 ** 27])
+
+
+def _epoch_jumps(name, capacity, layers, far):
     """A fixed sequence of steps alternating batch 16 (ragged) and batch 1 runs three times on the
     same inputs: from epoch 1000; across the 32-bit wrap; and with the epoch moved forward so that
-    every batch-16 step runs 65,536 or 65,535 epochs after the previous one (the slots of sequences
+    every batch-16 step runs one of the distances `far` after the previous one (the slots of sequences
     1..15 are not rewritten by the batch-1 steps in between).  All three give the same bits."""
     _need_gpu()
     from prime_kernels_amd import _native
 
     lib = _native.library()
     contexts = [40 + 37 * b for b in range(16)]
-    mod, model, embed, final_norm, lw, kv, cos_sin = _setup(16, contexts)
+    mod, model, embed, final_norm, lw, kv, cos_sin = _setup(16, contexts, layers, model=name, capacity=capacity)
     rt = mod.workspace(embed.device)
     stream = torch.cuda.current_stream().cuda_stream
     kv0 = [c.clone() for c in kv.caches]
@@ -137,7 +154,7 @@ def test_epoch_wrap_and_16_bit_jumps_with_alternating_batches():
         pos = list(contexts)
         outs = []
         last16 = None
-        jumps = [65536, 65535, 65536, 65535]
+        jumps = list(far)
         for k, B in enumerate(plan):
             if mode == "jump" and B == 16 and last16 is not None:
                 # the step epoch is the stored one + 1: make it last16 + jump
