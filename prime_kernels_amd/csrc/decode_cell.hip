@@ -49,9 +49,6 @@ constexpr uint32_t LDS_CU = 160u * 1024u;  // LDS of a CU (one workgroup each)
 #ifndef PK_CELL_DEPTH
 #define PK_CELL_DEPTH 4
 #endif
-#ifndef PK_CELL_UPL
-#define PK_CELL_UPL 4
-#endif
 #ifndef PK_CELL_TMIN
 #define PK_CELL_TMIN 8
 #endif
@@ -91,6 +88,7 @@ struct CG {
   static constexpr int TILES = E2E ? NT_MAX / R + IPC : (NT_MAX + R - NP - 1) / (R - NP);
   static constexpr int SCT = E2E ? TILES * 16 + IPC * 64 : (TILES * 16 + 63) / 64 * 64;
   static_assert(NP < R && NP <= 64, "a workgroup for every pair, a lane for every pair");
+  static_assert(NS <= NCW, "a wave for every sequence of the cell");
   static_assert(HU >= R && QU >= R && IU >= R, "rows of every projection for each workgroup (the producer divides by them)");
   static_assert(G::H % 64 == 0 && G::I % 64 == 0 && G::H % 4 == 0 && HU <= NCT, "whole k-steps and units");
   static_assert(G::V % (NWG * 16) == 0 && TL % NCW == 0, "LM-head tiles");
@@ -112,7 +110,7 @@ struct CW {
   static constexpr uint32_t V0 = BMAX * NWG;
   // UPL units of a vector per 64-byte line; consecutive lines of a vector lie SLOTS lines apart, so
   // that its lines spread over the memory channels
-  static constexpr uint32_t UPL = PK_CELL_UPL, LINES = (640 + UPL - 1) / UPL, SLOTS = BMAX * 5 + 1;
+  static constexpr uint32_t UPL = 4, LINES = (640 + UPL - 1) / UPL, SLOTS = BMAX * 5 + 1;
   static_assert(HU <= 640 && QU <= 640 && IU <= 640, "a vector's lines");
   static constexpr uint32_t REC0 = V0 + LINES * SLOTS * 4;
   static constexpr uint32_t REC = 66, END = REC0 + uint32_t(NWG) * IPW_MAX * REC;
@@ -169,7 +167,6 @@ struct SmemRest {
   int32_t sid[BMAX];                      // the cell's sequences by slot
   int32_t cs[BMAX];                       // every sequence's exchange slot
   int32_t ns, ni, ntile;
-  int32_t slow;                           // a workgroup with the longest chunk (-1: no pair has more than one)
   int32_t sS[BMAX], sPos[BMAX], sId[BMAX];
   long long sSlot[BMAX];
   float lm_val[NCW][BMAX];
@@ -315,15 +312,9 @@ __device__ __forceinline__ void setup(const Params& p, const PlanC<G, PX>& P, Sm
       sm.ntile = it.ntile;
     }
     const uint64_t m = __ballot(have);
-    float longest[1] = {on && C > 1 ? float((nt + C - 1) / C) : 0.f};
-    const float mine = longest[0];
-    wave_max_n<1>(longest);
-    const uint64_t sl = __ballot(mine > 0.f && mine == longest[0]);
-    const int slow = sl ? __shfl(r0 + C - 1, __ffsll((unsigned long long)sl) - 1) : -1;
     if (lane == 0) {
       sm.ni = m ? 1 : 0;
       if (!m) sm.ntile = 0;
-      sm.slow = slow;
     }
   }
 }
@@ -598,8 +589,10 @@ struct CC {
   }
 };
 
-// rsqrt(mean + eps): the hardware estimate (1 ulp) and one Newton step, a third of the instructions of a
-// correctly rounded square root and divide on a chain that runs 64 times a step.
+// rsqrt(mean + eps): the hardware estimate (1 ulp) and one Newton step, a third of the instructions of rms_scale's
+// square root and divide on a chain that runs 61 times a step (seven sequences: 566 us, 577 with rms_scale).  Over 2^26 sums
+// from 1e-6 to 1e9 it is nearer to 64 bits: mean error 0.43 to 0.47, worst 1.70 (times 2^-24); rms_scale 0.53 to
+// 0.55 and 2.36.
 template <int N>
 __device__ __forceinline__ float rms_rs(float sumsq) {
   const float m = fmaf(sumsq, 1.0f / float(N), 1e-5f);
@@ -647,45 +640,33 @@ __device__ __forceinline__ void norm_row(CC<G, PX>& C, const uint2 (&v)[CG<G, PX
     if (u < S::HU) *reinterpret_cast<uint2*>(C.sm.xs + q * S::XH + 4 * u) = norm4(v[j], nw.w[j], rs);
   }
 }
-// This workgroup's residual rows, from the units as norm_row takes them.
-template <int N, class G, int PX>
-__device__ __forceinline__ void keep_rows(CC<G, PX>& C, const uint2 (&v)[N][CG<G, PX>::LU]) {
-  using S = CG<G, PX>;
+// This workgroup's residual rows of the wave's sequence, from the units as norm_row takes them.
+template <class G, int PX>
+__device__ __forceinline__ void keep_rows(CC<G, PX>& C, const uint2 (&v)[CG<G, PX>::LU]) {
 #pragma unroll
-  for (int j = 0; j < S::LU; ++j) {
+  for (int j = 0; j < CG<G, PX>::LU; ++j) {
     const int u = C.lane + 64 * j;
-    if (u >= C.P.o0 && u < C.P.o1)
-#pragma unroll
-      for (int i = 0; i < N; ++i)
-        if (C.cw + NCW * i < C.ns) C.sm.res[C.cw + NCW * i][u - C.P.o0] = v[i][j];
+    if (u >= C.P.o0 && u < C.P.o1) C.sm.res[C.cw][u - C.P.o0] = v[j];
   }
 }
 
-// Wait for the cell's x or h1 vectors, keep this workgroup's residual rows, normalise.
-template <int N, class G, int PX>
+// Wait for the cell's x or h1 vectors (wave w: sequence w), keep this workgroup's residual rows, normalise.
+template <class G, int PX>
 __device__ __forceinline__ void stage_norm(CC<G, PX>& C, int kind, int l, const NormW<G, PX>& nw) {
   using S = CG<G, PX>;
-  u32x4 x[N * S::LU];
-  uint2 v[N][S::LU];
-  uint32_t live = 0;
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-    if (C.cw + NCW * i < C.ns) live |= ((1u << S::LU) - 1u) << (i * S::LU);
+  const bool mine = C.cw < C.ns;
+  u32x4 x[S::LU];
+  uint2 v[S::LU];
   const uint32_t o = CW<G>::vec_u(C.lane), oe = CW<G>::vec_u(min(C.lane, S::HU - 1 - 64 * (S::LU - 1)));
-  C.template poll<N * S::LU>(44 + kind, live, [&](const u32x4& u) { return C.vec_ok(u, l); },
-                             [&](int i) { return i % S::LU == S::LU - 1 ? oe : o; },
-                             [&](int i) {
-                               return CW<G>::vec_s(kind, C.slot0() + C.cw + NCW * (i / S::LU)) +
-                                      uint32_t(i % S::LU) * CW<G>::STRIDE64;
-                             }, x);
+  C.template poll<S::LU>(44 + kind, mine ? (1u << S::LU) - 1u : 0u, [&](const u32x4& u) { return C.vec_ok(u, l); },
+                         [&](int j) { return j == S::LU - 1 ? oe : o; },
+                         [&](int j) { return CW<G>::vec_s(kind, C.slot0() + C.cw) + uint32_t(j) * CW<G>::STRIDE64; }, x);
 #pragma unroll
-  for (int i = 0; i < N; ++i)
-#pragma unroll
-    for (int j = 0; j < S::LU; ++j) v[i][j] = make_uint2(x[i * S::LU + j].x, x[i * S::LU + j].y);
-  keep_rows<N>(C, v);
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-    if (C.cw + NCW * i < C.ns) norm_row(C, v[i], C.cw + NCW * i, nw);
+  for (int j = 0; j < S::LU; ++j) v[j] = make_uint2(x[j].x, x[j].y);
+  if (mine) {
+    keep_rows(C, v);
+    norm_row(C, v, C.cw, nw);
+  }
   C.cbar();
 }
 // The same for at most N sequences with thread t holding unit t of each: one load a sequence instead of
@@ -727,16 +708,15 @@ __device__ __forceinline__ void stage_norm_t(CC<G, PX>& C, int kind, int l, cons
 template <class G, int PX>
 __device__ __forceinline__ void stage_x(CC<G, PX>& C, int kind, int l, const NormW<G, PX>& nw) {
   if (C.ns <= 2) stage_norm_t<2>(C, kind, l, nw);
-  else if (C.ns <= NCW) stage_norm<1>(C, kind, l, nw);
-  else if constexpr (CG<G, PX>::NS > NCW) stage_norm<2>(C, kind, l, nw);
+  else stage_norm(C, kind, l, nw);
 }
 
 // Wait for the cell's attention vectors and stage them as rows of xs.
-template <int N, class G, int PX>
-__device__ __forceinline__ void stage_att_n(CC<G, PX>& C, int l) {
+template <class G, int PX>
+__device__ __forceinline__ void stage_att(CC<G, PX>& C) {
   using S = CG<G, PX>;
+  constexpr int N = S::NS, AU = G::H / 6;
   u32x4 x[N];
-  constexpr int AU = G::H / 6;
   const uint32_t o = CW<G>::vec_u(min(C.ct, AU - 1)), tg = C.tag, copy = C.copy;
   C.template poll<N>(44 + C_ATT, (1u << C.ns) - 1u, [&](const u32x4& u) { return u.w == tg; }, [&](int) { return o; },
                      [&](int i) { return CW<G>::vec_s(C_ATT, C.slot0() + i) + copy; }, x);
@@ -748,12 +728,6 @@ __device__ __forceinline__ void stage_att_n(CC<G, PX>& C, int l) {
         d[0] = x[i].x; d[1] = x[i].y; d[2] = x[i].z;
       }
   C.cbar();
-}
-template <class G, int PX>
-__device__ __forceinline__ void stage_att(CC<G, PX>& C, int l) {
-  if constexpr (CG<G, PX>::NS <= 4) stage_att_n<CG<G, PX>::NS>(C, l);
-  else if (C.ns <= 4) stage_att_n<4>(C, l);
-  else stage_att_n<8>(C, l);
 }
 
 template <int N, class G, int PX>
@@ -782,10 +756,7 @@ __device__ __forceinline__ void stage_act_n(CC<G, PX>& C, int l) {
 template <class G, int PX>
 __device__ __forceinline__ void stage_act(CC<G, PX>& C, int l) {
   if (C.ns <= 2) stage_act_n<2>(C, l);
-  else if constexpr (CG<G, PX>::NS > 2) {
-    if (C.ns <= 4) stage_act_n<4>(C, l);
-    else if constexpr (CG<G, PX>::NS > 4) stage_act_n<8>(C, l);
-  }
+  else stage_act_n<CG<G, PX>::NS>(C, l);
 }
 
 // One projection phase: D[row][sequence] = W x over this workgroup's `groups` 8-row groups (NT 16-row
@@ -1194,7 +1165,7 @@ __device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
   if (w == 2 && Cc > 1 && ng > 0) {
     const uint32_t ou = uint32_t(2 + 2 * g0 + min(lane, 2 * ng - 1)) * 16u;
     float v[3] = {0.f, 0.f, 0.f};
-    constexpr int N = 13;  // a sequence alone in its cell has up to 25 chunks a head
+    constexpr int N = 13;  // a sequence alone in its cell has up to 21 chunks a head
     for (int c0 = 0; c0 < Cc; c0 += N) {
       u32x4 y[N];
       const int nc = min(N, Cc - c0);
@@ -1580,20 +1551,15 @@ __device__ __forceinline__ void consumer(const Params& p, const PlanC<G, PX>& P,
     }
   const int seq = col < C.ns ? sm.sid[col] : 0;  // global sequence of this lane's column
   // layer 0's x: the embedding rows
-  auto first_x = [&](auto nn, const NormW<G, PX>& nw) {
-    constexpr int N = decltype(nn)::value;
-    uint2 v[N][S::LU];
+  auto first_x = [&](const NormW<G, PX>& nw) {
+    if (C.cw < C.ns) {
+      const uint2* row = reinterpret_cast<const uint2*>(p.embed + size_t(sm.sId[sm.sid[C.cw]]) * G::H);
+      uint2 v[S::LU];
 #pragma unroll
-    for (int i = 0; i < N; ++i)
-#pragma unroll
-      for (int j = 0; j < S::LU; ++j)
-        v[i][j] = C.cw + NCW * i < C.ns && C.lane + 64 * j < S::HU
-                      ? *(reinterpret_cast<const uint2*>(p.embed + size_t(sm.sId[sm.sid[C.cw + NCW * i]]) * G::H) + C.lane + 64 * j)
-                      : make_uint2(0u, 0u);
-    keep_rows<N>(C, v);
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-      if (C.cw + NCW * i < C.ns) norm_row(C, v[i], C.cw + NCW * i, nw);
+      for (int j = 0; j < S::LU; ++j) v[j] = C.lane + 64 * j < S::HU ? row[C.lane + 64 * j] : make_uint2(0u, 0u);
+      keep_rows(C, v);
+      norm_row(C, v, C.cw, nw);
+    }
     C.cbar();
   };
   for (int l = 0; l < p.n_layers && C.ns > 0; ++l) {
@@ -1603,7 +1569,7 @@ __device__ __forceinline__ void consumer(const Params& p, const PlanC<G, PX>& P,
     tr(l, 0);
     const NormW<G, PX> nw1(C);
     const Weights<S::KSH, S::TQ, G, PX> wq(C, (4 * nuq + 7) / 8);
-    if (l == 0) first_x(std::integral_constant<int, (S::NS + NCW - 1) / NCW>{}, nw1);
+    if (l == 0) first_x(nw1);
     else stage_x(C, C_X, l - 1, nw1);
     tr(l, 1);
     {
@@ -1658,7 +1624,7 @@ __device__ __forceinline__ void consumer(const Params& p, const PlanC<G, PX>& P,
       }
     };
     const Weights<S::KSH, S::TO, G, PX> wo(C, (4 * nuo + 7) / 8);
-    stage_att(C, l);
+    stage_att(C);
     tr(l, 9);
     {
       floatx4 acc[S::TO];
