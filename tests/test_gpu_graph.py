@@ -14,15 +14,15 @@ def _need_gpu():
         pytest.skip("no GPU")
 
 
-def _setup(batch, ctxs, seed=7, layers=4):
+def _setup(batch, ctxs, seed=7, layers=4, model="decode_megakernel_360m", capacity=None):
     import prime_kernels_amd as pk
     from prime_kernels_amd import workload as WL
 
-    mod = pk.load("decode_megakernel_360m")
+    mod = pk.load(model)
     model = mod.MODEL
     dev = torch.device("cuda:0")
     embed, final_norm, lw = WL.random_weights(model, seed, dev, layers=layers)
-    cap = max(ctxs) + 64
+    cap = capacity or max(ctxs) + 64
     kv = WL.PagedKV(model, batch, cap, layers=layers, device=dev, seed=seed + 1, fill="randn")
     cos_sin = WL.rope_table(cap, device=dev)
     st = dict(
@@ -61,9 +61,25 @@ def test_decode_step_replays_from_a_graph(batch, launch):
         lib.pk_set_option(_native.PK_OPT_COOPERATIVE, old)
 
 
-def _replay_check(batch):
+@pytest.mark.parametrize("launch", ["ordinary", "cooperative"])
+@pytest.mark.parametrize("batch,layers,capacity", [(3, 4, None), (7, 3, None), (8, 4, 7696)],
+                         ids=["b3", "b7_odd_layers", "b8_end_to_end"])
+def test_135m_batched_step_replays_from_a_graph(batch, layers, capacity, launch):
+    """135M's batched kernel, on both splits of its attention (8 * 7,696 tokens are past 61,440)."""
+    _need_gpu()
+    from prime_kernels_amd import _native
+
+    lib = _native.library()
+    old = lib.pk_set_option(_native.PK_OPT_COOPERATIVE, 1 if launch == "cooperative" else 0)
+    try:
+        _replay_check(batch, layers=layers, model="decode_megakernel", capacity=capacity)
+    finally:
+        lib.pk_set_option(_native.PK_OPT_COOPERATIVE, old)
+
+
+def _replay_check(batch, **setup):
     ctxs = [300 + 97 * b for b in range(batch)]
-    mod, kv, st, logits, kw = _setup(batch, ctxs)
+    mod, kv, st, logits, kw = _setup(batch, ctxs, **setup)
     kv0 = [c.clone() for c in kv.caches]
     _fill(kv, st, [5] * batch, ctxs)
     mod.decode_step(**kw)                       # first use of the device: outside capture

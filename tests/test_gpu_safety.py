@@ -28,6 +28,8 @@ def _need_gpu():
 
 
 MODELS = {"360m": "decode_megakernel_360m", "135m": "decode_megakernel"}
+# 135M's batched kernel: sequences, and the block table's capacity (past 61,440 tokens in all: the end-to-end split)
+CELLS = {"cells": (3, None), "cells_full": (16, None), "cells_end_to_end": (8, 7696)}
 
 
 def _setup(batch_max, contexts, layers=2, seed=5, model="360m", capacity=None):
@@ -60,7 +62,7 @@ def _step(mod, embed, final_norm, lw, kv, cos_sin, ids, positions):
 
 
 @pytest.mark.parametrize("report", ["next_call", "check_failures"])
-@pytest.mark.parametrize("path", ["split_role", "split_wide", "general", "batched"])
+@pytest.mark.parametrize("path", ["split_role", "split_wide", "general", "batched", *CELLS])
 def test_abandoned_wait_poisons_outputs_and_is_reported(path, report):
     """The failed step is reported once: by the next decode call (which launches nothing), or by
     check_failures, after which the next call runs normally (split_wide: a context past the narrow
@@ -69,9 +71,10 @@ def test_abandoned_wait_poisons_outputs_and_is_reported(path, report):
     from prime_kernels_amd import _native
 
     lib = _native.library()
-    batch = 3 if path == "batched" else 1
+    batch, capacity = CELLS.get(path, (3 if path == "batched" else 1, None))
     contexts = [3000] if path == "split_wide" else [300 + 41 * b for b in range(batch)]
-    mod, model, embed, final_norm, lw, kv, cos_sin = _setup(batch, contexts)
+    mod, model, embed, final_norm, lw, kv, cos_sin = _setup(batch, contexts, model="135m" if path in CELLS else "360m",
+                                                            capacity=capacity)
     rt = mod.workspace(embed.device)
     stream = torch.cuda.current_stream().cuda_stream
     old = lib.pk_set_option(_native.PK_OPT_SPLIT_ROLE, 0 if path == "general" else 1)
@@ -238,7 +241,7 @@ def test_attention_records_through_uncached_memory_give_the_same_bits(split_role
         lib.pk_set_option(_native.PK_OPT_SPLIT_ROLE, old_sr)
 
 
-@pytest.mark.parametrize("case", ["b1_split_role", "b1_split_wide", "b1_general", "b16_ragged"])
+@pytest.mark.parametrize("case", ["b1_split_role", "b1_split_wide", "b1_general", "b16_ragged", *CELLS])
 def test_arrival_skew_leaves_every_bit_unchanged(case):
     """Arrival-skew test of the tagged exchange protocol: with PK_OPT_SKEW every workgroup sleeps a
     pseudo-random 0..23 x 512 cycles (from the seed, the workgroup, the layer and the site) before each
@@ -249,9 +252,12 @@ def test_arrival_skew_leaves_every_bit_unchanged(case):
     from prime_kernels_amd import _native
 
     lib = _native.library()
-    batch = 16 if case == "b16_ragged" else 1
+    batch, capacity = CELLS.get(case, (16 if case == "b16_ragged" else 1, None))
     contexts = [40 + 53 * b for b in range(batch)] if batch > 1 else [3000] if case == "b1_split_wide" else [900]
-    mod, model, embed, final_norm, lw, kv, cos_sin = _setup(batch, contexts)
+    if case in CELLS:
+        contexts[1] = 1400                                    # a pair in several chunks
+    mod, model, embed, final_norm, lw, kv, cos_sin = _setup(batch, contexts, 4 if case in CELLS else 2,
+                                                            model="135m" if case in CELLS else "360m", capacity=capacity)
     kv0 = [c.clone() for c in kv.caches]
     ids = [(11 + 97 * b) % 49152 for b in range(batch)]
     old_sr = lib.pk_set_option(_native.PK_OPT_SPLIT_ROLE, 0 if case == "b1_general" else 1)
@@ -307,7 +313,7 @@ def test_exchange_units_are_never_torn(mode, slot):
     assert checked == rounds * participants * participants * 4, checked
 
 
-@pytest.mark.parametrize("path", ["split_role", "split_wide", "general", "batched", "mxfp8", "mxfp8_general"])
+@pytest.mark.parametrize("path", ["split_role", "split_wide", "general", "batched", "mxfp8", "mxfp8_general", *CELLS])
 def test_cooperative_launch_gives_the_same_bits(path):
     """The decode kernels run with the ordinary launch by default; PK_OPT_COOPERATIVE (or
     PK_LAUNCH=cooperative) launches them with hipLaunchCooperativeKernel as the reference does
@@ -316,9 +322,10 @@ def test_cooperative_launch_gives_the_same_bits(path):
     from prime_kernels_amd import _native
 
     lib = _native.library()
-    batch = 3 if path == "batched" else 1
+    batch, capacity = CELLS.get(path, (3 if path == "batched" else 1, None))
     contexts = [2100] if path.startswith("mxfp8") or path == "split_wide" else [300 + 41 * b for b in range(batch)]
-    mod, model, embed, final_norm, lw, kv, cos_sin = _setup(batch, contexts)
+    mod, model, embed, final_norm, lw, kv, cos_sin = _setup(batch, contexts, model="135m" if path in CELLS else "360m",
+                                                            capacity=capacity)
     if path.startswith("mxfp8"):
         import prime_kernels_amd as pk
         from prime_kernels_amd import mxfp8
