@@ -102,7 +102,6 @@ struct CG {
 // read in a format it was not written in): the workgroups' end records per sequence (tag: epoch), the
 // vectors per sequence (tag: epoch, and the layer in the word before it; the attention vector: CC::tag), the
 // attention records of each workgroup's items (statistics, 2 units; partial sums, 64 units; CC::tag).
-// The vectors and records are there twice, the second copy for some attentions' units (CC::copy).
 enum CKind { C_X, C_ATT, C_H1, C_QKV, C_ACT };
 template <class G>
 struct CW {
@@ -113,8 +112,8 @@ struct CW {
   static constexpr uint32_t UPL = 4, LINES = (640 + UPL - 1) / UPL, SLOTS = BMAX * 5 + 1;
   static_assert(HU <= 640 && QU <= 640 && IU <= 640, "a vector's lines");
   static constexpr uint32_t REC0 = V0 + LINES * SLOTS * 4;
-  static constexpr uint32_t REC = 66, END = REC0 + uint32_t(NWG) * IPW_MAX * REC;
-  static constexpr uint32_t COPY = END - V0, TOTAL = END + COPY;
+  static constexpr uint32_t REC = 66;
+  static constexpr uint32_t TOTAL = REC0 + uint32_t(NWG) * IPW_MAX * REC;
   __device__ static uint32_t end(int b, int wg) { return (uint32_t(b) * NWG + uint32_t(wg)) * 16u; }
   // unit u of vector `kind` of sequence slot cs (cell * NS + slot): lane part and uniform part
   __device__ static uint32_t vec_u(int u) { return (V0 + uint32_t(u) / UPL * SLOTS * 4u + uint32_t(u) % UPL) * 16u; }
@@ -504,15 +503,14 @@ struct CC {
   __device__ __forceinline__ void refresh() { asm volatile("" : "+v"(lane), "+v"(ct)); }
   // The attention's units hold three payload words and one for the epoch and the layer.  Every unit that a step uses
   // is written and read by the same waves in each of its layers, so from a step's second layer on only the layer
-  // before it has to be told apart: odd layers flip the epoch's top bit.  At its first use in a step a unit may be
-  // as old as the program, so a step leaves none with the bit flipped: a last layer that is odd takes the second copy.
-  // The first use of either copy then finds whole epochs of other steps, as with the units that hold both words.
-  // (A step that gave up may leave a flipped one.)
-  uint32_t tag = 0, copy = 0;
+  // before it has to be told apart: the top bits of the epoch, flipped in turn, do that.  At its first use in a step a
+  // unit may be as old as the program, so the first and the last layer have the epoch as it is, and a first use finds
+  // whole epochs of other steps, as with the units that hold both words.  (A step of two layers, or one that gave up,
+  // leaves flipped ones, which pass as another step's after 2^30 steps at the earliest.)
+  uint32_t tag = 0;
   __device__ __forceinline__ void begin_layer(int l) {
-    const bool odd = l & 1, last = l == p.n_layers - 1;
-    tag = epoch ^ (odd && !last ? 0x80000000u : 0u);
-    copy = odd && last ? W::COPY * 16u : 0u;
+    const bool whole = l == 0 || (l == p.n_layers - 1 && l > 1);
+    tag = epoch ^ (whole ? 0u : l & 1 ? 1u << 31 : 1u << 30);
   }
   __device__ __forceinline__ uint32_t filled() const {
     typedef __attribute__((address_space(3))) const volatile u32x4 lds_u32x4;
@@ -717,9 +715,9 @@ __device__ __forceinline__ void stage_att(CC<G, PX>& C) {
   using S = CG<G, PX>;
   constexpr int N = S::NS, AU = G::H / 6;
   u32x4 x[N];
-  const uint32_t o = CW<G>::vec_u(min(C.ct, AU - 1)), tg = C.tag, copy = C.copy;
+  const uint32_t o = CW<G>::vec_u(min(C.ct, AU - 1)), tg = C.tag;
   C.template poll<N>(44 + C_ATT, (1u << C.ns) - 1u, [&](const u32x4& u) { return u.w == tg; }, [&](int) { return o; },
-                     [&](int i) { return CW<G>::vec_s(C_ATT, C.slot0() + i) + copy; }, x);
+                     [&](int i) { return CW<G>::vec_s(C_ATT, C.slot0() + i); }, x);
   if (C.ct < AU)
 #pragma unroll
     for (int i = 0; i < N; ++i)
@@ -916,7 +914,7 @@ __device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
   const int slot = C.slot0() + one(it.slot);
   const int nquad = (nt + 3) / 4;
   const int me = C.P.cell * S::R + C.P.r;
-  const uint32_t tg = C.tag, copy = C.copy;
+  const uint32_t tg = C.tag;
   const uint32_t kpos = C.pos, vpos = kpos + uint32_t(nt) * 2u * PKT;
   C.pos = vpos + uint32_t(nt) * 2u * PKT;
   const bool has_new = w == NCW - 1 && one(it.leader);  // the new token is wave 3's, in the chunk with the pair's end
@@ -1028,13 +1026,13 @@ __device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
       if (lane < 2)
         C.st(W::rec(me, 0, lane),
              lane == 0 ? u32x4{__float_as_uint(M[0]), __float_as_uint(M[1]), __float_as_uint(M[2]), tg}
-                       : u32x4{__float_as_uint(inv[0]), __float_as_uint(inv[1]), __float_as_uint(inv[2]), tg}, copy);
+                       : u32x4{__float_as_uint(inv[0]), __float_as_uint(inv[1]), __float_as_uint(inv[2]), tg});
     }
     tr(5);
     u32x4 y[2];
     const uint32_t o = W::rec(r0 + min(lane, Cc - 1), 0, 0);
     C.template poll<2>(51, 3u, [&](const u32x4& u) { return u.w == tg; }, [&](int i) { return o + 16u * uint32_t(i); },
-                       [&](int) { return copy; }, y);
+                       [&](int) { return 0u; }, y);
     const bool mine = lane < Cc;
     float mk[3];
 #pragma unroll
@@ -1135,7 +1133,7 @@ __device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
   C.release(C.pos);
   C.cbar();
   // ---- publish (wave 0): a pair in one chunk gives its attention values, others their fp32 partial sums ----
-  const uint32_t att = W::vec_s(C_ATT, slot) + copy;
+  const uint32_t att = W::vec_s(C_ATT, slot);
   if (w == 0) {
     skew_delay(p.skew, C.P.wg, l, 15);
     if (Cc > 1) {
@@ -1146,7 +1144,7 @@ __device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
 #pragma unroll
         for (int j = 0; j < NCW; ++j) v[i] += wo[j * 192 + 3 * lane + i];
       }
-      C.st(W::rec(me, 0, 2 + lane), u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), tg}, copy);
+      C.st(W::rec(me, 0, 2 + lane), u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), tg});
     } else if (lane < GRP) {
       float v[6];
 #pragma unroll
@@ -1170,7 +1168,7 @@ __device__ __forceinline__ void attention_one(CC<G, PX>& C, int l) {
       u32x4 y[N];
       const int nc = min(N, Cc - c0);
       C.template poll<N>(52, (1u << nc) - 1u, [&](const u32x4& u) { return u.w == tg; }, [&](int) { return ou; },
-                         [&](int i) { return W::rec(r0 + c0 + i, 0, 0) + copy; }, y);
+                         [&](int i) { return W::rec(r0 + c0 + i, 0, 0); }, y);
 #pragma unroll
       for (int i = 0; i < N; ++i)
         if (i < nc) {
@@ -1198,7 +1196,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
   SmemC<G, PX>& sm = C.sm;
   const int lane = C.lane, w = C.cw;
   const int ni = __builtin_amdgcn_readfirstlane(sm.ni), ntile = __builtin_amdgcn_readfirstlane(sm.ntile);
-  const uint32_t tg = C.tag, copy = C.copy;
+  const uint32_t tg = C.tag;
   const int wgkey = C.P.cell * S::R;
   const uint32_t kpos = C.pos, vpos = kpos + uint32_t(ntile) * 2u * PKT;
   C.pos = vpos + uint32_t(ntile) * 2u * PKT;
@@ -1330,7 +1328,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
     if (sm.it[k].C > 1) {
       const u32x4 um = {__float_as_uint(rl(mx, 0)), __float_as_uint(rl(mx, 4)), __float_as_uint(rl(mx, 8)), tg};
       const u32x4 ul = {__float_as_uint(rl(ex, 0)), __float_as_uint(rl(ex, 4)), __float_as_uint(rl(ex, 8)), tg};
-      if (lane < 2) C.st(W::rec(wgkey + C.P.r, k, lane), lane == 0 ? um : ul, copy);
+      if (lane < 2) C.st(W::rec(wgkey + C.P.r, k, lane), lane == 0 ? um : ul);
     } else if (lane < 12 && (lane & 3) == 0) {
       sm.at.gml[k][lane >> 2] = mx;
       sm.at.gml[k][3 + (lane >> 2)] = 1.0f / ex;
@@ -1347,7 +1345,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) off[i] = int(W::rec(wgkey + r0 + c, c == 0 ? k0 : 0, i));
       C.template poll<2>(51, 3u, [&](const u32x4& u) { return u.w == tg; }, [&](int i) { return uint32_t(off[i]); },
-                         [&](int) { return copy; }, x);
+                         [&](int) { return 0u; }, x);
       const bool mine = lane < Cc;
       float M[3], mk[3], lk[3];
 #pragma unroll
@@ -1476,7 +1474,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
 #pragma unroll
         for (int x = 0; x < NCW; ++x) v[i] += o[x * 192 + 3 * lane + i];
       }
-      C.st(W::rec(wgkey + C.P.r, k, 2 + lane), u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), tg}, copy);
+      C.st(W::rec(wgkey + C.P.r, k, 2 + lane), u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), tg});
     } else if (lane < 32) {
       float v[6];
 #pragma unroll
@@ -1486,7 +1484,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
         for (int x = 0; x < NCW; ++x) v[i] += o[x * 192 + 6 * lane + i];
       }
       C.st(W::vec_u(sm.it[k].g * 32 + lane) + W::vec_s(C_ATT, slot0 + sm.it[k].slot),
-           u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), tg}, copy);
+           u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), tg});
     }
   }
   tr(7);
@@ -1506,7 +1504,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
         u32x4 x[N];
         const int n = min(N, Cc - c0);
         C.template poll<N>(52, (1u << n) - 1u, [&](const u32x4& u) { return u.w == tg; }, [&](int) { return o; },
-                           [&](int i) { return W::rec(r0 + c0 + i, c0 + i == 0 ? k0 : 0, 0) + copy; }, x);
+                           [&](int i) { return W::rec(r0 + c0 + i, c0 + i == 0 ? k0 : 0, 0); }, x);
 #pragma unroll
         for (int i = 0; i < N; ++i)
           if (i < n) {
@@ -1520,7 +1518,7 @@ __device__ __forceinline__ void attention_many(CC<G, PX>& C, int l) {
       for (int i = 0; i < 3; ++i) y[i] = dpp<0xb1>(0.f, v[i]);  // the pair's other lane
       if ((lane & 1) == 0 && lane < 2 * ng)
         C.st(W::vec_u(sm.it[k].g * 32 + g0 + (lane >> 1)) + W::vec_s(C_ATT, slot0 + sm.it[k].slot),
-             u32x4{pack2(v[0], v[1]), pack2(v[2], y[0]), pack2(y[1], y[2]), tg}, copy);
+             u32x4{pack2(v[0], v[1]), pack2(v[2], y[0]), pack2(y[1], y[2]), tg});
     }
   }
   C.cbar();  // the attention buffers share storage with the staged rows

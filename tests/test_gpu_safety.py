@@ -10,7 +10,7 @@
 * Exchange words carry the full 32-bit step epoch: steps that alternate batch sizes (so some words
   are not rewritten every step) give the same bits across the epoch's 32-bit wrap and across jumps
   of 65,536 and 65,535 epochs, where a 16-bit tag (with or without a skipped zero) would accept a
-  stale word as current; 135M's batched kernel also across jumps of 2^27 and 2^31 epochs, where a tag of
+  stale word as current; 135M's batched kernel also across jumps of 2^27 to 2^31 epochs, where a tag of
   (epoch << 5) | layer would.  (decode_kernel_b's softmax statistics and partial sums carry such a tag.)
 """
 
@@ -125,12 +125,13 @@ def test_epoch_wrap_and_16_bit_jumps_with_alternating_batches():
     _epoch_jumps("360m", None, 2, [65536, 65535, 65536, 65535])
 
 
-@pytest.mark.parametrize("layers", [1, 2, 3])
+@pytest.mark.parametrize("layers", [1, 2, 3, 4])
 @pytest.mark.parametrize("capacity", [None, 3904], ids=["whole_workgroups", "end_to_end"])
 def test_epoch_wrap_and_long_jumps_of_the_cell_kernel(capacity, layers):
     """Both splits of 135M's batched kernel (16 * 3,904 tokens of block table are past 61,440), with a last
-    layer of either parity (the attention's units say the layer by one bit)."""
-    _epoch_jumps("135m", capacity, layers, [2 ** 27, 65535, 2 ** 31, 2 ** 27])
+    layer of either parity (the attention's units say the layer by two bits of the epoch, which a step of two
+    layers leaves flipped)."""
+    _epoch_jumps("135m", capacity, layers, [2 ** 27, 65535, 2 ** 30, 2 ** 27 if layers == 2 else 2 ** 31])
 
 
 def _epoch_jumps(name, capacity, layers, far):
