@@ -3602,11 +3602,13 @@ static int decode_impl(void* stream, int B, int n_layers, const void* input_ids,
         }
         return PK_OK;
       }
-      // 135M, three or more: cells of XCDs, each decoding its own sequences (seven sequences of 100..2000 tokens:
-      // 588 us against 1,191 here).  The cells sum in another order, and one rounding that falls the other way
-      // travels through the layers: the logits of the two kernels, both as far from 64-bit arithmetic, are 0.017 to
-      // 0.026 apart (relative norm, six seeds) for 135M and 0.022 to 0.038 for 360M.  More than 0.03 is not taken for
-      // speed, so 360M stays here (four sequences: 1,388 us, 731 on cells; sixteen: 1,644 and 1,106).
+      // 135M, three or more: cells of XCDs, each decoding its own sequences (seven sequences of 60..1900 tokens:
+      // 602 us against 1,192 here).  The cells sum in another order, and one rounding that falls the other way
+      // travels through the layers.  Neither kernel is nearer to 64-bit arithmetic (135M, three layers, 40 seeds: the
+      // cells' error is larger by 0.04 to 0.12 % +- 0.1 %), but their logits are 0.017 to 0.026 apart (relative norm,
+      // six seeds) after 135M's 30 layers and 0.022 to 0.038 after 360M's 32.  A step's results were not to move
+      // by more than 0.03 for speed, so 360M stays here (four sequences: 1,388 us, 731 on cells of four XCDs;
+      // sixteen: 1,644 and 1,106).
       if constexpr (G::H == 576)
         if (B > 2 && !input_hidden)
           return cell_launch(p, reinterpret_cast<const uint8_t*>(state->ws) + cell_region_off(), s, opt_cooperative());

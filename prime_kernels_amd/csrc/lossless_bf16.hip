@@ -191,7 +191,7 @@ __global__ void __launch_bounds__(256) lz_clear(uint64_t* states, uint32_t* tick
 // gives up, which its successors take over, so that the layer ends disabled with a total of ~0.
 // 32 layers of random weights (315 MB read, 236 MB written) take 168 us (3.3 TB/s), a call 219; counting
 // first and placing the escapes in a later kernel took 98 + 5 + 67 (scattered 4-byte header writes, a second
-// read of the escaped chunks), a call 257, and three launches and a copy for each layer 621.
+// read of the escaped chunks), a call 257, and three launches and a copy for each layer 540 to 645, by the host.
 __global__ void __launch_bounds__(64 * kWavesPerBlock) lz_encode_many(BatchArgs a) {
   __shared__ uint32_t ticket, before_block, wave_count[kWavesPerBlock];
   const LayerArgs L = a.l[blockIdx.y];
